@@ -31,7 +31,7 @@ LIB = os.path.join(PKG, "liblaya.so")
 HOST_LIB = os.path.join(PKG, "liblaya_host.so")
 TOOLS = {"laya-parity": "laya_parity.cpp", "laya-bench": "laya_bench.cpp"}
 
-HIP_SOURCES = ["engine.hip", "kernels_gemm.hip", "kernels_attn.hip", "kernels_norm.hip"]
+HIP_SOURCES = ["engine.hip", "kernels_gemm.hip", "kernels_gemm_small.hip", "kernels_attn.hip", "kernels_norm.hip"]
 CPP_SOURCES = ["model.cpp", "pack.cpp"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-fPIC", "-std=c++17", "-I" + CSRC, "-I" + INCLUDE,

@@ -35,6 +35,7 @@
 #include <vector>
 
 #include "common.h"
+#include "gemm_small.h"
 #include "kernels.h"
 #include "laya_api.h"
 #include "laya_ext.h"
@@ -656,10 +657,11 @@ struct Engine : EngineIface {
                    (g.ln_mr ? 1 : 0) + (g.stats ? 2 : 0) + (g.bias ? 4 : 0));
   }
 
-  // one GEMM of the pass: listed while the pass is collected for tuning, otherwise launched with
-  // the measured configuration of its bucket (the analytic planner's where none was measured)
+  // one GEMM of the pass: listed while the pass is collected for tuning, otherwise launched on the
+  // few-row kernel where its rule takes it (same bits, nothing to tune), else with the measured configuration of its bucket (the analytic planner's where none was measured)
   void gemm(int epi, GemmArgs g, hipStream_t st) {
     if (collecting) { collecting->emplace_back(epi, g); return; }
+    if (pin_cfg < 0 && launch_gemm_small<T>(epi, g, st)) return;
     if (pin_cfg >= 0) {
       g.cfg = pin_cfg; g.split_rows = pin_split; g.cfg_tail = pin_tail;
     } else {
@@ -756,7 +758,7 @@ struct Engine : EngineIface {
     collecting = nullptr;
     for (auto& eg : list) {
       const TuneKey key = tune_key(eg.first, eg.second);
-      if (eg.second.ksplit <= 1 && !tuned.count(key)) tuned[key] = tune_gemm(eg.first, eg.second);
+      if (eg.second.ksplit <= 1 && !gemm_small_takes<T>(eg.first, eg.second) && !tuned.count(key)) tuned[key] = tune_gemm(eg.first, eg.second);
     }
     LAYA_HIP(hipStreamSynchronize(stream));
     tuned_shapes.insert(s);
@@ -1064,6 +1066,7 @@ int laya_ext_prof_sequence(void* h, int* stages, int cap) {
 }
 static float* g_ext_ws = nullptr;          // split-K workspace of laya_ext_gemm (caller's memory)
 static size_t g_ext_ws_bytes = 0;
+static int g_ext_ks = 0;                   // split-K factor pinned with it
 
 // The measurement hooks run inside the caller's process, which shares the HIP runtime (and its
 // per-thread last error) with the caller: a stale error that the caller's own HIP calls left must
@@ -1115,8 +1118,12 @@ int laya_ext_gemm(int dtype, int epi, const void* A, const void* W, void* C, con
   hipEvent_t a, b;
   if (ms) { LAYA_HIP(hipEventCreate(&a)); LAYA_HIP(hipEventCreate(&b)); LAYA_HIP(hipEventRecord(a, st)); }
   for (int i = 0; i < iters; i++) {
-    if (dtype == 0) launch_gemm<float>(epi == 0 ? EPI_STORE : EPI_RESID, g, st);
-    else launch_gemm<bf16_t>(epi == 0 ? EPI_STORE : EPI_RESID, g, st);
+    const int e = epi == 0 ? EPI_STORE : EPI_RESID;
+    if (dtype == 0) {
+      if (!launch_gemm_small<float>(e, g, st)) launch_gemm<float>(e, g, st);
+    } else if (g_ext_ks > 1 || !launch_gemm_small<bf16_t>(e, g, st)) {
+      launch_gemm<bf16_t>(e, g, st);
+    }
   }
   if (ms) {
     LAYA_HIP(hipEventRecord(b, st));
@@ -1174,6 +1181,7 @@ int laya_ext_gemm_ksplit(int ks, void* ws, size_t ws_bytes) {
   if (ks < 0 || ks > 64 || (ks > 1 && (!ws || ws_bytes == 0))) return -2;
   g_ext_ws = static_cast<float*>(ws);
   g_ext_ws_bytes = ws_bytes;
+  g_ext_ks = ks;
   return laya::gemm_pin_ksplit(ks);
 }
 }  // extern "C"

@@ -1,0 +1,102 @@
+"""The few-row GEMM kernel (kernels_gemm_small.hip) against the large tiles, on the GPU.
+
+bf16: every output must have the bits of the large-tile kernel (a pinned tile configuration keeps a
+launch there), whatever variant its rule picks: sizes on both sides of the 16-, 32-, 64- and 128-row
+tiles, K of one stage, an odd number of stages and more stages than the ring holds, N that a tile does
+not divide, and the rule's own upper ends.  fp32: the same rows inside a call too large for the rule.
+Rows past M (a guard behind C) must stay untouched.  Whole passes, with the QKV, GeGLU and split-K
+epilogues the hook does not reach: one question in an engine pinned to a large tile and in the default
+one, and in fp32 alone and inside a batch."""
+import numpy as np
+import pytest
+
+from layamd_amd import checkpoint as ck
+from layamd_amd import engine as le
+from layamd_amd import workloads as wl
+
+pytestmark = pytest.mark.gpu
+
+SHAPES = [(1, 1024, 1024), (31, 1024, 64), (33, 72, 192), (64, 8, 128), (65, 4096, 1024), (127, 1024, 2624),
+          (129, 768, 1152), (200, 1024, 2624), (255, 5248, 1024), (257, 3072, 768), (513, 1024, 4096),
+          (1024, 1024, 1024), (1025, 1024, 2624)]
+
+
+def _operands(M, N, K, dtype, seed):
+    import torch
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    t = torch.bfloat16 if dtype == "bf16" else torch.float32
+    A = torch.randn(M, K, generator=g, device="cuda").to(t)
+    W = (torch.randn(N, K, generator=g, device="cuda") * 0.02).to(t)
+    b = torch.randn(N, generator=g, device="cuda")
+    X = torch.randn(M + 8, N, generator=g, device="cuda")
+    return A, W, b, X
+
+
+def _all(lib, A, W, b, X):
+    """Plain store, bias + ReLU, bias + GELU, residual with and without bias; 8 guard rows behind each."""
+    import torch
+    M, N = A.shape[0], W.shape[0]
+    out = []
+    for bias, act in ((None, 0), (b, 1), (b, 2)):
+        C = torch.full((M + 8, N), 7.0, dtype=A.dtype, device="cuda")
+        le.gemm(lib, A, W, C, bias=bias, act=act)
+        out.append(C)
+    for bias in (None, b):
+        C = X.clone()
+        le.gemm(lib, A, W, C, bias=bias, residual=True)
+        out.append(C)
+    torch.cuda.synchronize()
+    return out
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_bf16_bits_of_the_large_tiles(M, N, K):
+    import torch
+    lib = le.load_library()
+    ops = _operands(M, N, K, "bf16", M + N + K)
+    prev = le.gemm_config(lib, 3)
+    try:
+        want = _all(lib, *ops)
+        le.gemm_config(lib, -1)
+        got = _all(lib, *ops)
+    finally:
+        le.gemm_config(lib, prev)
+    for w, g in zip(want, got):
+        assert torch.isfinite(g[:M].float()).all()
+        assert torch.equal(w, g)
+    assert all((g[M:] == 7.0).all() for g in got[:3]) and torch.equal(got[3][M:], ops[3][M:])
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_fp32_rows_of_a_larger_call(M, N, K):
+    import torch
+    lib = le.load_library()
+    A, W, b, X = _operands(M, N, K, "fp32", M + N + K)
+    got = _all(lib, A, W, b, X)
+    reps = 8192 // M + 1                                  # the same rows over and over, past the rule's range
+    big = _all(lib, A.repeat(reps, 1), W, b, torch.cat([X[:M].repeat(reps, 1), X[M:]]))
+    for w, g in zip(big, got):
+        assert torch.isfinite(g[:M]).all()
+        assert torch.equal(w[:M], g[:M])
+    assert all((g[M:] == 7.0).all() for g in got[:3]) and torch.equal(got[3][M:], X[M:])
+
+
+@pytest.mark.parametrize("preset,lens", [("large", [16]), ("large", [128]), ("large", [300, 77]), ("large", [512, 400, 333]),
+                                         ("base", [41]), ("base", [200, 260])])
+def test_bf16_passes_of_a_pinned_engine(preset, lens):
+    d = ck.cached_checkpoint(preset, ln_jitter=0.05)
+    b = wl.make_batch(ck.PRESETS[preset], lens, [5] * len(lens), seed=len(lens))
+    env = {"LAYA_MAX_TOKENS": 4096, "LAYA_GRAPHS": 0}
+    want = le.Engine(None, d, precision="bf16", env=dict(env, LAYA_GEMM_CFG=3)).forward_flat(*b.flat())
+    got = le.Engine(None, d, precision="bf16", env=env).forward_flat(*b.flat())
+    assert np.isfinite(want[0]).all() and np.array_equal(want[0], got[0]) and np.array_equal(want[1], got[1])
+
+
+def test_fp32_question_alone_and_in_a_batch():
+    b = wl.c3(0)
+    e = le.Engine(None, ck.cached_checkpoint("large", ln_jitter=0.05), precision="fp32", env={"LAYA_MAX_TOKENS": 16384, "LAYA_GRAPHS": 0})
+    logits, act = e.forward_flat(*b.flat())
+    at = np.concatenate([[0], np.cumsum(b.nmark)])
+    for i in (0, 7, int(np.argmin(b.lens)), int(np.argmax(b.lens))):
+        lo, ac = e.forward_flat(*b.subset([i]).flat())
+        assert np.array_equal(lo, logits[at[i]:at[i + 1]]) and np.array_equal(ac[0], act[i]), i
