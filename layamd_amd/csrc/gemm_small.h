@@ -4,9 +4,9 @@
 
 namespace laya {
 
-// Runs the GEMM on the few-row kernel when its rule takes the shape (rows few enough that the large
-// tiles of launch_gemm leave most of the chip idle, aligned operands, no LayerNorm fold) and returns
-// true; otherwise launches nothing and returns false.  Every output is the one launch_gemm gives, bit
+// Runs the GEMM on the few-row kernel when its rule takes the shape (bf16: rows few enough that the
+// large tiles of launch_gemm leave most of the chip idle; fp32: any number; aligned operands, no
+// LayerNorm fold) and returns true; otherwise launches nothing and returns false.  Every output is the one launch_gemm gives, bit
 // for bit: the K order, the split-K chunks (GemmArgs::ksplit) and the epilogue's arithmetic are the
 // same.  A pinned tile configuration (gemm_config) keeps launch_gemm.
 template <typename T>

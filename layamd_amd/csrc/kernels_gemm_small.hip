@@ -396,9 +396,9 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_small(const GemmArgs a, i
 }
 
 // ---------------------------------------------------------------- variants and rule
-// Tiles, smallest first.  The step and ring depths use what LDS holds beside the vmcnt limit: 96 to
-// 144 KB, one workgroup per CU, but for fp32's 64x64 tile (80 KB, two per CU), whose loop is bound by
-// the fp32 MFMA rate and not by the fills.
+// Tiles, smallest first.  bf16: the step and ring depths use what LDS holds, 96 to 144 KB, one workgroup
+// per CU.  fp32 (but for the smallest tile, whose grid is at most one per CU): 72 to 80 KB, two per CU,
+// because the loop is bound by the fp32 MFMAs, and a second workgroup's fill the gaps around barriers.
 struct SmallTile { int bm, bn; };
 static SmallTile small_tile(int v) {
   static const SmallTile t[kSmallVariants] = {{32, 16}, {32, 32}, {32, 64}, {64, 64}, {128, 64}};
@@ -435,8 +435,14 @@ template <typename T>
 void launch_gemm_small_variant(int epi, const GemmArgs& a, int v, hipStream_t st) {
   switch (v) {
     case 0: launch_small<T, 32, 16, 2, 1, 2, 8>(epi, a, st); return;
-    case 1: launch_small<T, 32, 32, 2, 2, 2, 8>(epi, a, st); return;
-    case 2: launch_small<T, 32, 64, 2, 2, 2, 6>(epi, a, st); return;
+    case 1:
+      if constexpr (sizeof(T) == 2) launch_small<T, 32, 32, 2, 2, 2, 8>(epi, a, st);
+      else launch_small<T, 32, 32, 2, 2, 1, 10>(epi, a, st);
+      return;
+    case 2:
+      if constexpr (sizeof(T) == 2) launch_small<T, 32, 64, 2, 2, 2, 6>(epi, a, st);
+      else launch_small<T, 32, 64, 2, 2, 1, 6>(epi, a, st);
+      return;
     case 3:
       if constexpr (sizeof(T) == 2) launch_small<T, 64, 64, 2, 4, 2, 4>(epi, a, st);
       else launch_small<T, 64, 64, 2, 2, 1, 5>(epi, a, st);
@@ -504,13 +510,29 @@ static int small_cus() {
 //   QKV, N 3072, K 1024:       M 128 6.7 | 13.6   256 7.5 | 13.4   512 10.0 | 13.4   768 17.2 | 13.6
 //   GeGLU, N 5248, K 1024:     M 64 6.9 | 8.6     192 7.4 | 8.9    256 9.8 | 9.5
 //   split-K, N 1024, K 4096:   M 128 9.4 | 15.7   512 16.3 | 21.1  1024 21.0 | 37.8  2048 31.4 | 74.8
+// fp32 is bound by the fp32 MFMA rate, so there the rule weighs the tiles of the busiest CU, at any M:
+//   N 1024, K 2624, residual:  M 128 15.3 | 59.2   512 28.4 | 58.6   1031 64.9 | 104   9664 406 | 678
+//   QKV, N 3072, K 1024:       M 128 13.9 | 28.6   512 32.9 | 44.1   1031 67.3 | 81.6  9664 477 | 564
+// (9664 x 1024 x 2624: 128 of the 152 TFLOP/s that a large fp32 product reaches on this chip).
 // 128x64 tiles only gain where the large tiles have none (QKV needs BM <= BN there) or write partial
 // products to memory (split-K; there also in more than one round).
 template <typename T>
 int gemm_small_pick(int epi, const GemmArgs& a) {
   if (gemm_pinned() >= 0) return -1;
-  if constexpr (sizeof(T) == 4) return -1;
   const int cus = small_cus();
+  if constexpr (sizeof(T) == 4) {
+    // relative time of the busiest CU: its tiles times their area, by the tile's cost per area at load
+    static const double cost[4] = {0.125 * 1.9, 0.25 * 1.25, 0.5 * 1.08, 1.0};
+    int best = -1;
+    double bt = 0;
+    for (int v = 0; v < 4; v++) {
+      const SmallTile t = small_tile(v);
+      const int64_t tiles = (int64_t)((a.M + t.bm - 1) / t.bm) * ((a.N + t.bn - 1) / t.bn);
+      const double c = (double)((tiles + cus - 1) / cus) * cost[v];
+      if ((best < 0 || c < bt) && gemm_small_fits<T>(epi, a, v)) { best = v; bt = c; }
+    }
+    return best;
+  }
   for (int v = 0; v < kSmallVariants; v++) {
     const SmallTile t = small_tile(v);
     const int64_t tiles = (int64_t)((a.M + t.bm - 1) / t.bm) * ((a.N + t.bn - 1) / t.bn);

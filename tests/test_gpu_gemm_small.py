@@ -3,7 +3,7 @@
 bf16: every output must have the bits of the large-tile kernel (a pinned tile configuration keeps a
 launch there), whatever variant its rule picks: sizes on both sides of the 16-, 32-, 64- and 128-row
 tiles, K of one stage, an odd number of stages and more stages than the ring holds, N that a tile does
-not divide, and the rule's own upper ends.  fp32: the same rows inside a call too large for the rule.
+not divide, and the rule's own upper ends.  fp32: those of the generic kernel.
 Rows past M (a guard behind C) must stay untouched.  Whole passes, with the QKV, GeGLU and split-K
 epilogues the hook does not reach: one question in an engine pinned to a large tile and in the default
 one, and in fp32 alone and inside a batch."""
@@ -67,18 +67,26 @@ def test_bf16_bits_of_the_large_tiles(M, N, K):
     assert all((g[M:] == 7.0).all() for g in got[:3]) and torch.equal(got[3][M:], ops[3][M:])
 
 
-@pytest.mark.parametrize("M,N,K", SHAPES)
-def test_fp32_rows_of_a_larger_call(M, N, K):
+@pytest.mark.parametrize("M,N,K", SHAPES + [(2500, 1024, 1024), (4096, 768, 768)])
+def test_fp32_bits_of_the_generic_kernel(M, N, K):
+    """An output 4 bytes off its alignment keeps the generic kernel."""
     import torch
     lib = le.load_library()
     A, W, b, X = _operands(M, N, K, "fp32", M + N + K)
-    got = _all(lib, A, W, b, X)
-    reps = 8192 // M + 1                                  # the same rows over and over, past the rule's range
-    big = _all(lib, A.repeat(reps, 1), W, b, torch.cat([X[:M].repeat(reps, 1), X[M:]]))
-    for w, g in zip(big, got):
-        assert torch.isfinite(g[:M]).all()
-        assert torch.equal(w[:M], g[:M])
-    assert all((g[M:] == 7.0).all() for g in got[:3]) and torch.equal(got[3][M:], X[M:])
+
+    def off(t):
+        o = torch.empty(t.numel() + 1, device="cuda")[1:].view(t.shape)
+        return o.copy_(t)
+
+    for bias, act, residual in ((None, 0, False), (b, 1, False), (b, 2, False), (None, 0, True), (b, 0, True)):
+        start = X if residual else torch.full((M + 8, N), 7.0, device="cuda")
+        got, want = start.clone(), off(start)
+        assert want.data_ptr() % 16 == 4
+        le.gemm(lib, A, W, got, bias=bias, act=act, residual=residual)
+        le.gemm(lib, A, W, want, bias=bias, act=act, residual=residual)
+        torch.cuda.synchronize()
+        assert torch.isfinite(got[:M]).all()
+        assert torch.equal(got, want)
 
 
 @pytest.mark.parametrize("preset,lens", [("large", [16]), ("large", [128]), ("large", [300, 77]), ("large", [512, 400, 333]),
