@@ -1,21 +1,6 @@
 // Attention over packed variable-length sequences for gfx950 (wave64 MFMA, fp32 online softmax).
-// Two kernels: k_attention_bf16 (the bf16 engine's, described above it) and k_attention<T>, the
-// fp32 engine's, described here.
-//
-// One 256-thread workgroup owns one query tile (<= 64 queries of one sequence) of one head;
-// each wave64 owns 16 queries.  Keys advance in blocks of 64: the workgroup stages the block's
-// K rows ([key][d], 16-byte chunks XOR-swizzled by key) and V^T rows ([d][key], swizzled by d)
-// in LDS, then every wave computes
-//
-//     S^T = K Q^T    (MFMA A = K rows, B = Q rows, both d-contiguous)
-//     O^T += V^T P^T (MFMA A = V^T rows from LDS, B = P^T straight from the S^T registers)
-//
-// Working in the transposed frame keeps one query per lane column (lane l holds query l % 16):
-// the 16x16 accumulator layout puts S^T[key 4*(l/16)+i][query l%16] in lane l, which is exactly
-// the B-operand layout P^T needs for the next MFMA, with keys relabelled consistently in the
-// V^T operand, so P never goes through LDS.  Row max / row sum need only two cross-lane steps
-// (lanes l, l^16, l^32, l^48 share a query).  Scores and the running max/sum are fp32; the
-// score matrix never touches memory.
+// Two kernels: k_attention_bf16 (the bf16 engine's, described above it) and k_attention_f32, the
+// fp32 engine's.
 //
 // Masks: key j of the sequence is visible to query position p when j < len and, for sliding
 // layers, |p - j| <= window_half (inclusive, HF masking_utils.py:141-151).  Keys beyond the
@@ -32,191 +17,231 @@ typedef float f32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));   // one 16-byte chunk
 typedef uint32_t u32x2_t __attribute__((ext_vector_type(2)));   // 8 bytes
 
-template <typename T>
-__global__ __launch_bounds__(256) void k_attention(const T* __restrict__ Q, const T* __restrict__ K, int ldqk,
-                                                   const T* __restrict__ Vt, int ldv, T* __restrict__ O, int ldo,
-                                                   const AttnTile* __restrict__ tiles, const int* __restrict__ soff,
-                                                   const int* __restrict__ vlen, const int* __restrict__ gq,
-                                                   const int* __restrict__ grow,
-                                                   int window_half, float scale) {
-  constexpr int HD = 64;
-  constexpr int CPR = HD * (int)sizeof(T) / 16;        // 16-byte chunks per 64-element row
-  constexpr int EPC = 16 / (int)sizeof(T);             // elements per chunk
-  __shared__ u32x4_t Ks[64 * CPR];                       // [key][chunk ^ (key % CPR)]
-  __shared__ u32x4_t Vs[64 * CPR];                       // [d][...] swizzled by d
+// max and sum over lanes l, l ^ 16, l ^ 32, l ^ 48
+__device__ __forceinline__ float quad_rows_max(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(a[0]), __uint_as_float(a[1]));
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(b[0]), __uint_as_float(b[1]));
+}
+__device__ __forceinline__ float quad_rows_sum(float v) {
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+}
 
-  const AttnTile tile = tiles[blockIdx.x];
-  if (tile.nq <= 0) return;                              // an empty tile of the pass's tile capacity
-  const int h = blockIdx.y;
+// ======================================================================================
+// fp32 attention (v_mfma_f32_16x16x4_f32).  A workgroup of four waves owns a query tile of one head;
+// keys advance in blocks of 64, staged in LDS (K rows [key][d], 16-byte chunks XOR-swizzled by key, V^T
+// rows [d][key], swizzled by d).  A wave works on 16 queries and the 32 keys of one half of the block:
+//
+//     S^T = K Q^T    (MFMA A = K rows, B = Q rows, both d-contiguous)
+//     O^T += V^T P^T (MFMA A = V^T rows from LDS, B = P^T straight from the S^T registers)
+//
+// In the transposed frame a lane column is a query (lane l holds query l % 16): the accumulator layout
+// puts S^T[key 4 (l / 16) + i][query l % 16] in lane l, which is the B operand of the next product.
+//
+// The lower and the upper halves of the blocks are two classes of keys with a running maximum, sum and
+// output each, joined at the end.  SPLIT: 32 queries per workgroup, a wave per 16 queries and class, and
+// two buffers per operand, so that the next block's loads are in flight under this one's products.
+// Otherwise 64 queries, each wave both classes of its 16, one buffer (more workgroups per CU hide the
+// loads).  Blocks and classes are counted from the question's first key, and a half block out of a
+// query's range adds exact zeros and moves no maximum: both forms give the same bits, in any tiling.
+//
+// What bounds it: the fp32 MFMAs (4096 cycles for 64 queries and 64 keys on one CU), and for a few
+// questions, whose 64-query tiles do not fill the CUs, the chain over the keys; SPLIT halves the chain.
+// Two questions of 112 and 318 tokens, 16 heads: 19.8 us with this kernel's predecessor (whole tiles, one
+// class), 11.8 now; 32 questions, 9953 tokens: 184 -> 152 (sliding 84 -> 74).  Keys on four waves with
+// operands straight from L2 had a quarter of the chain, but L2 bound it at 25 B a cycle and CU (12.3 us and
+// 200 us on the same).
+// ======================================================================================
+template <bool SPLIT>
+__global__ __launch_bounds__(256) void k_attention_f32(const float* __restrict__ Q, const float* __restrict__ K, int ldqk,
+                                                       const float* __restrict__ Vt, int ldv, float* __restrict__ O, int ldo,
+                                                       const AttnTile* __restrict__ tiles, const int* __restrict__ soff,
+                                                       const int* __restrict__ vlen, const int* __restrict__ gq,
+                                                       const int* __restrict__ grow, int window_half, float scale) {
+  constexpr int NQ = SPLIT ? 32 : 64, NB = SPLIT ? 2 : 1, NC = SPLIT ? 1 : 2;
+  __shared__ f32x4_t Ks[NB][64 * 16], Vs[NB][64 * 16];
+
+  // heads are the fastest grid dimension: with H a multiple of 8 a head's K and V^T stay in one XCD's L2
+  AttnTile tile = tiles[SPLIT ? blockIdx.y >> 1 : blockIdx.y];
+  const int sub = SPLIT ? (int)(blockIdx.y & 1) * 32 : 0;
+  if (sub >= tile.nq) return;                            // (also an empty tile of the pass's tile capacity)
+  tile.q0 += sub;
+  tile.nq = min(tile.nq - sub, NQ);
+  const int h = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
-  const int b = tile.seq, len = vlen[b], base = soff[b], vb = base;   // V^T column = row
+  const int b = tile.seq, len = vlen[b], base = soff[b];
 
-  // this lane's query (16 per wave)
-  const int r = wave * 16 + l16;
+  // this lane's query and the keys it sees, [jlo, jhi)
+  const int r = (SPLIT ? wave >> 1 : wave) * 16 + l16;
   const bool qvalid = r < tile.nq;
   const int rr = qvalid ? r : 0;
   int p, orow;
   if (gq) { const int gi = gq[tile.q0 + rr]; p = grow[gi] - base; orow = gi; }
   else { p = tile.q0 + rr; orow = base + p; }
+  const bool win = window_half > 0 && !gq;
+  const int jlo = win ? max(0, p - window_half) : 0, jhi = win ? min(len, p + window_half + 1) : len;
+  // keys of the tile
+  const int lo = win ? max(0, tile.q0 - window_half) : 0;
+  const int hi = win ? min(len, tile.q0 + tile.nq + window_half) : len;
 
-  // key range of the tile
-  int lo = 0, hi = len;
-  if (window_half > 0 && !gq) {
-    lo = max(0, tile.q0 - window_half) & ~15;
-    hi = min(len, tile.q0 + tile.nq - 1 + window_half + 1);
+  f32x4_t qf[4];                                         // Q[p][16 g + 4 c ..]
+  const f32x4_t* qrow = reinterpret_cast<const f32x4_t*>(Q + (size_t)(base + p) * ldqk + h * 64);
+#pragma unroll
+  for (int c = 0; c < 4; c++) qf[c] = qrow[4 * g + c];
+
+  struct State { f32x4_t o[4]; float mc, l; } s[NC];     // output, running max times c2, this lane's part of the sum
+#pragma unroll
+  for (int c = 0; c < NC; c++) {
+#pragma unroll
+    for (int db = 0; db < 4; db++) s[c].o[db] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    s[c].mc = -INFINITY;
+    s[c].l = 0.f;
   }
+  const float c2 = scale * 1.44269504088896340736f;
 
-  // Q fragments (B operand of S^T = K Q^T): lane holds Q[p][...] chunks
-  const T* qrow = Q + (size_t)(base + p) * ldqk + h * HD;
-  u32x4_t qf[4];
-  if constexpr (sizeof(T) == 2) {
-    qf[0] = reinterpret_cast<const u32x4_t*>(qrow)[g];          // d = 8g .. 8g+7
-    qf[1] = reinterpret_cast<const u32x4_t*>(qrow)[4 + g];      // d = 32 + 8g ..
-  } else {
+  // block k0 to registers (thread: chunk tid % 16 of rows tid / 16 + 16 it) and from there to LDS
+  const int sr = tid >> 4, sc = tid & 15;
+  f32x4_t rk[4], rv[4];
+  auto fetch = [&](int k0) {
 #pragma unroll
-    for (int c = 0; c < 4; c++) qf[c] = reinterpret_cast<const u32x4_t*>(qrow)[4 * g + c];   // d = 16g + 4c ..
-  }
-
-  f32x4_t o[4];
-#pragma unroll
-  for (int db = 0; db < 4; db++) o[db] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-  float m_run = -INFINITY, l_run = 0.f;
-
-  for (int k0 = lo; k0 < hi; k0 += 64) {
-    // ---- stage K rows and V^T rows of keys [k0, k0 + 64) ----
-#pragma unroll
-    for (int it = 0; it < (64 * CPR) / 256; it++) {
-      const int idx = tid + it * 256;
-      const int kr = idx / CPR, ch = idx % CPR;
-      const int key = min(k0 + kr, len - 1);
-      Ks[kr * CPR + (ch ^ (kr % CPR))] =
-          reinterpret_cast<const u32x4_t*>(K + (size_t)(base + key) * ldqk + h * HD)[ch];
-      const int d = kr;                                  // V^T row d, chunk ch covers keys ch*EPC ..
-      const u32x4_t v = *reinterpret_cast<const u32x4_t*>(Vt + (size_t)(h * HD + d) * ldv + vb + k0 + ch * EPC);
-      if constexpr (sizeof(T) == 2) {
-        // 8-byte units (4 keys) swizzled by d so 16 lanes reading 16 rows hit distinct banks
-        u32x2_t* vrow = reinterpret_cast<u32x2_t*>(&Vs[d * CPR]);
-        vrow[(2 * ch) ^ (d & 15)] = (u32x2_t){v.x, v.y};
-        vrow[(2 * ch + 1) ^ (d & 15)] = (u32x2_t){v.z, v.w};
-      } else {
-        Vs[d * CPR + (ch ^ (d & 15))] = v;
-      }
+    for (int it = 0; it < 4; it++) {
+      const int key = min(k0 + sr + 16 * it, len - 1);
+      rk[it] = reinterpret_cast<const f32x4_t*>(K + (size_t)(base + key) * ldqk + h * 64)[sc];
+      rv[it] = *reinterpret_cast<const f32x4_t*>(Vt + (size_t)(h * 64 + sr + 16 * it) * ldv + base + k0 + 4 * sc);
     }
-    __syncthreads();
-
-    // ---- S^T = K Q^T for 4 sub-blocks of 16 keys ----
-    f32x4_t st[4];
+  };
+  auto stage = [&](int buf) {
 #pragma unroll
-    for (int kb = 0; kb < 4; kb++) {
-      st[kb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-      const int kr = kb * 16 + l16;
-      if constexpr (sizeof(T) == 2) {
-#pragma unroll
-        for (int s = 0; s < 2; s++) {
-          const u32x4_t kf = Ks[kr * CPR + ((4 * s + g) ^ (kr % CPR))];
-          st[kb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf),
-                                                           __builtin_bit_cast(bf16x8_t, qf[s]), st[kb], 0, 0, 0);
-        }
-      } else {
-#pragma unroll
-        for (int c = 0; c < 4; c++) {
-          const f32x4_t kf = __builtin_bit_cast(f32x4_t, Ks[kr * CPR + ((4 * g + c) ^ (kr % CPR))]);
-          const f32x4_t qv = __builtin_bit_cast(f32x4_t, qf[c]);
-#pragma unroll
-          for (int u = 0; u < 4; u++) st[kb] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u], qv[u], st[kb], 0, 0, 0);
-        }
-      }
+    for (int it = 0; it < 4; it++) {
+      Ks[buf][(sr + 16 * it) * 16 + (sc ^ sr)] = rk[it];
+      Vs[buf][(sr + 16 * it) * 16 + (sc ^ sr)] = rv[it];
     }
+  };
 
-    // ---- mask, online softmax (lane-local query; 4 lane groups share it) ----
+  // the 32 keys of class cls of the block at k0: scores, online softmax, output
+  auto half = [&](State& a, int buf, int k0, int cls) {
+    const int kc = k0 + 32 * cls;
+    if (kc >= hi || kc + 32 <= lo) return;
+    const f32x4_t *ks = &Ks[buf][32 * cls * 16], *vs = Vs[buf];
+    f32x4_t st[2];
+#pragma unroll
+    for (int n = 0; n < 2; n++) st[n] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+      f32x4_t kf[2];
+#pragma unroll
+      for (int n = 0; n < 2; n++) kf[n] = ks[(16 * n + l16) * 16 + ((4 * g + c) ^ l16)];
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int n = 0; n < 2; n++) st[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[n][u], qf[c][u], st[n], 0, 0, 0);
+    }
     float mx = -INFINITY;
 #pragma unroll
-    for (int kb = 0; kb < 4; kb++)
+    for (int n = 0; n < 2; n++)
 #pragma unroll
       for (int i = 0; i < 4; i++) {
-        const int j = k0 + kb * 16 + 4 * g + i;
-        const bool ok = j < len && (window_half == 0 || abs(p - j) <= window_half);
-        const float v = ok ? st[kb][i] * scale : -INFINITY;
-        st[kb][i] = v;
+        const int j = kc + 16 * n + 4 * g + i;
+        const float v = j >= jlo && j < jhi ? st[n][i] : -INFINITY;
+        st[n][i] = v;
         mx = fmaxf(mx, v);
       }
-    mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-    mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-    const float m_new = fmaxf(m_run, mx);
-    float alpha = 1.f, rs = 0.f;
-    if (m_new != -INFINITY) {
-      alpha = __expf(m_run - m_new);
+    const float m_new = fmaxf(a.mc, quad_rows_max(mx) * c2);
+    const float mz = m_new == -INFINITY ? 0.f : m_new;   // nothing visible yet: every exp2 below is 0
+    const float alpha = __builtin_amdgcn_exp2f(a.mc - mz);
+    a.mc = m_new;
+    float rs = 0.f;
 #pragma unroll
-      for (int kb = 0; kb < 4; kb++)
+    for (int n = 0; n < 2; n++)
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-          const float e = st[kb][i] == -INFINITY ? 0.f : __expf(st[kb][i] - m_new);
-          st[kb][i] = e;
-          rs += e;
-        }
-    } else {
-#pragma unroll
-      for (int kb = 0; kb < 4; kb++) st[kb] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-    }
-    rs += __shfl_xor(rs, 16, 64);
-    rs += __shfl_xor(rs, 32, 64);
-    l_run = l_run * alpha + rs;
-    m_run = m_new;
-#pragma unroll
-    for (int db = 0; db < 4; db++) o[db] *= alpha;
-
-    // ---- O^T += V^T P^T ----
-    if constexpr (sizeof(T) == 2) {
-#pragma unroll
-      for (int t = 0; t < 2; t++) {
-        // B operand: keys 32t + 4g + (0..3) and 32t + 16 + 4g + (0..3) of this lane's query
-        bf16x8_t pb;
-#pragma unroll
-        for (int i = 0; i < 4; i++) {
-          pb[i] = (__bf16)st[2 * t][i];
-          pb[4 + i] = (__bf16)st[2 * t + 1][i];
-        }
-#pragma unroll
-        for (int db = 0; db < 4; db++) {
-          const int d = db * 16 + l16;
-          const u32x2_t* vrow = reinterpret_cast<const u32x2_t*>(&Vs[d * CPR]);
-          const u32x2_t u0 = vrow[(8 * t + g) ^ (d & 15)];
-          const u32x2_t u1 = vrow[(8 * t + 4 + g) ^ (d & 15)];
-          const u32x4_t va = (u32x4_t){u0.x, u0.y, u1.x, u1.y};
-          o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, va), pb, o[db], 0, 0, 0);
-        }
+      for (int i = 0; i < 4; i++) {
+        const float e = __builtin_amdgcn_exp2f(fmaf(st[n][i], c2, -mz));
+        st[n][i] = e;
+        rs += e;
       }
-    } else {
+    a.l = fmaf(a.l, alpha, rs);
 #pragma unroll
-      for (int kb = 0; kb < 4; kb++)
+    for (int db = 0; db < 4; db++) a.o[db] *= alpha;
 #pragma unroll
-        for (int db = 0; db < 4; db++) {
-          const int d = db * 16 + l16;
-          const f32x4_t va = __builtin_bit_cast(f32x4_t, Vs[d * CPR + ((4 * kb + g) ^ (d & 15))]);  // keys 16kb+4g+0..3
+    for (int n = 0; n < 2; n++) {
+      f32x4_t vf[4];                                     // V^T[16 db + l16][keys kc + 16 n + 4 g ..]
 #pragma unroll
-          for (int u = 0; u < 4; u++) o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[u], st[kb][u], o[db], 0, 0, 0);
-        }
+      for (int db = 0; db < 4; db++) vf[db] = vs[(16 * db + l16) * 16 + ((8 * cls + 4 * n + g) ^ l16)];
+#pragma unroll
+      for (int u = 0; u < 4; u++)
+#pragma unroll
+        for (int db = 0; db < 4; db++) a.o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[db][u], st[n][u], a.o[db], 0, 0, 0);
+    }
+  };
+
+  int k0 = lo & ~63;
+  if constexpr (SPLIT) {
+    fetch(k0);
+    stage(0);
+    if (k0 + 64 < hi) fetch(k0 + 64);
+    __syncthreads();
+    for (int buf = 0; k0 < hi; k0 += 64, buf ^= 1) {
+      half(s[0], buf, k0, wave & 1);
+      if (k0 + 64 < hi) {
+        stage(buf ^ 1);                                  // last read before the previous barrier
+        if (k0 + 128 < hi) fetch(k0 + 128);
+      }
+      __syncthreads();
+    }
+  } else {
+    for (; k0 < hi; k0 += 64) {
+      fetch(k0);
+      stage(0);
+      __syncthreads();
+      half(s[0], 0, k0, 0);
+      half(s[NC - 1], 0, k0, 1);
+      __syncthreads();
+    }
+  }
+
+  // the two classes together: the upper half's state into x
+  State x = s[NC - 1];
+  if constexpr (SPLIT) {
+    f32x4_t* os = Ks[0];
+    float* ml = reinterpret_cast<float*>(Vs[0]);
+    const int at = (wave >> 1) * 64 + lane;
+    if (wave & 1) {
+#pragma unroll
+      for (int db = 0; db < 4; db++) os[db * 128 + at] = s[0].o[db];
+      ml[at] = s[0].mc;
+      ml[128 + at] = s[0].l;
     }
     __syncthreads();
+    if (wave & 1) return;
+#pragma unroll
+    for (int db = 0; db < 4; db++) x.o[db] = os[db * 128 + at];
+    x.mc = ml[at];
+    x.l = ml[128 + at];
   }
-
+  const float mj = fmaxf(s[0].mc, x.mc), mz = mj == -INFINITY ? 0.f : mj;
+  const float f0 = __builtin_amdgcn_exp2f(s[0].mc - mz), f1 = __builtin_amdgcn_exp2f(x.mc - mz);
+  const float l = quad_rows_sum(fmaf(x.l, f1, s[0].l * f0));
   if (!qvalid) return;
-  // o[db][i] = O^T[d = 16db + 4g + i][query]; write 4 consecutive d per block
-  const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-  T* orow_p = O + (size_t)orow * ldo + h * HD;
+  // o[db][i] = O^T[d = 16 db + 4 g + i][query]
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  float* orow_p = O + (size_t)orow * ldo + h * 64;
 #pragma unroll
   for (int db = 0; db < 4; db++) {
-    const int d = db * 16 + 4 * g;
-    if constexpr (sizeof(T) == 2) {
-      u32x2_t u;
-      u[0] = (uint32_t)f2bf(o[db][0] * inv) | ((uint32_t)f2bf(o[db][1] * inv) << 16);
-      u[1] = (uint32_t)f2bf(o[db][2] * inv) | ((uint32_t)f2bf(o[db][3] * inv) << 16);
-      *reinterpret_cast<u32x2_t*>(orow_p + d) = u;
-    } else {
-      *reinterpret_cast<float4*>(orow_p + d) = make_float4(o[db][0] * inv, o[db][1] * inv, o[db][2] * inv, o[db][3] * inv);
-    }
+    f32x4_t v;
+#pragma unroll
+    for (int i = 0; i < 4; i++) v[i] = fmaf(x.o[db][i], f1, s[0].o[db][i] * f0) * inv;
+    *reinterpret_cast<f32x4_t*>(orow_p + 16 * db + 4 * g) = v;
   }
 }
+
+// Workgroups of whole tiles (tiles times heads) up to which the split form runs: about one per CU.  Split
+// against whole tiles, us, 16 heads: 2 tiles 8.3 | 8.8 (both near the time of a launch), 7 tiles 11.8 | 17.7,
+// 13 tiles 13.2 | 14.9, 16 tiles of one question 49.4 | 50.5, 46 tiles 57.0 | 48.7, 173 tiles 197 | 152.
+constexpr int64_t kAttnF32Split = 256;
 
 __device__ __forceinline__ uint32_t lds_addr_a(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
@@ -616,8 +641,12 @@ void launch_attention(const T* Q, const T* K, int ldqk, int kv_rows, const T* Vt
       LAYA_LAUNCH(k_attention_bf16<2>, dim3(H, ntiles), dim3(128), 0, st, Q, K, ldqk, kv_rows, Vt, ldv, H * 64, O,
                          ldo, tiles, soff, vlen, gq, grow, window_half, scale);
   } else {
-    LAYA_LAUNCH((k_attention<T>), dim3(ntiles, H), dim3(256), 0, st, Q, K, ldqk, Vt, ldv, O, ldo, tiles, soff,
-                       vlen, gq, grow, window_half, scale);
+    if ((int64_t)ntiles * H <= kAttnF32Split)
+      LAYA_LAUNCH(k_attention_f32<true>, dim3(H, ntiles * 2), dim3(256), 0, st, Q, K, ldqk, Vt, ldv, O, ldo, tiles, soff, vlen,
+                  gq, grow, window_half, scale);
+    else
+      LAYA_LAUNCH(k_attention_f32<false>, dim3(H, ntiles), dim3(256), 0, st, Q, K, ldqk, Vt, ldv, O, ldo, tiles, soff, vlen,
+                  gq, grow, window_half, scale);
   }
 }
 

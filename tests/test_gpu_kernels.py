@@ -289,6 +289,29 @@ def test_attention_gathered_queries(dtype):
         moff += len(m)
 
 
+@pytest.mark.parametrize("window_half", [0, 64, 7, 100])
+def test_attention_fp32_split_and_whole_tiles(window_half):
+    """The fp32 kernel's two forms: a batch whose tiles fill the CUs (whole 64-query tiles) and each of its
+    questions alone (32-query workgroups, the keys of a block on two waves) give the same bits, against
+    the fp64 oracle, with windows that are no multiple of a block too; without a window also as gathered
+    queries."""
+    pk = Packed(EDGE_LENS + [33, 31, 700, 1024], 16, "fp32", seed=15)
+    tiles = pk.encoder_tiles(64)
+    whole = pk.run(tiles, window_half)
+    rows = [np.arange(pk.soff[b], pk.soff[b] + L) for b, L in enumerate(pk.lens)]
+    for b, L in enumerate(pk.lens):
+        alone = pk.run(np.ascontiguousarray(tiles[(tiles[:, 0] == b) & (tiles[:, 2] > 0)]), window_half)
+        assert np.array_equal(alone[rows[b]], whole[rows[b]]), (b, L)
+        _check(pk, whole[rows[b]], b, np.arange(L), window_half, False)
+    if window_half == 0:
+        grow = np.concatenate(rows).astype(np.int32)
+        at = np.concatenate([[0], np.cumsum(pk.lens)])
+        gt = tiles.copy()
+        gt[:, 1] += at[gt[:, 0]].astype(np.int32)
+        gathered = pk.run(gt, 0, gq=np.arange(len(grow), dtype=np.int32), grow=grow, out_rows=len(grow))
+        assert np.array_equal(gathered, whole[grow])
+
+
 def test_attention_rejects_bad_arguments():
     """The hook refuses what the kernels cannot take (128-query tiles in fp32 or gathered mode,
     misaligned strides) before launching anything."""
