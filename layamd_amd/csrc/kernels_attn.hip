@@ -34,27 +34,27 @@ __device__ __forceinline__ float quad_rows_sum(float v) {
 // ======================================================================================
 // fp32 attention (v_mfma_f32_16x16x4_f32).  A workgroup of four waves owns a query tile of one head;
 // keys advance in blocks of 64, staged in LDS (K rows [key][d], 16-byte chunks XOR-swizzled by key, V^T
-// rows [d][key], swizzled by d).  A wave works on 16 queries and the 32 keys of one half of the block:
+// rows [d][key], swizzled by d):
 //
 //     S^T = K Q^T    (MFMA A = K rows, B = Q rows, both d-contiguous)
 //     O^T += V^T P^T (MFMA A = V^T rows from LDS, B = P^T straight from the S^T registers)
 //
 // In the transposed frame a lane column is a query (lane l holds query l % 16): the accumulator layout
 // puts S^T[key 4 (l / 16) + i][query l % 16] in lane l, which is the B operand of the next product.
-//
-// The lower and the upper halves of the blocks are two classes of keys with a running maximum, sum and
-// output each, joined at the end.  SPLIT: 32 queries per workgroup, a wave per 16 queries and class, and
-// two buffers per operand, so that the next block's loads are in flight under this one's products.
-// Otherwise 64 queries, each wave both classes of its 16, one buffer (more workgroups per CU hide the
-// loads).  Blocks and classes are counted from the question's first key, and a half block out of a
-// query's range adds exact zeros and moves no maximum: both forms give the same bits, in any tiling.
+// Row max and row sum need two cross-lane steps (lanes l, l ^ 16, l ^ 32, l ^ 48 share a query).
 //
 // What bounds it: the fp32 MFMAs (4096 cycles for 64 queries and 64 keys on one CU), and for a few
-// questions, whose 64-query tiles do not fill the CUs, the chain over the keys; SPLIT halves the chain.
-// Two questions of 112 and 318 tokens, 16 heads: 19.8 us with this kernel's predecessor (whole tiles, one
-// class), 11.8 now; 32 questions, 9953 tokens: 184 -> 152 (sliding 84 -> 74).  Keys on four waves with
-// operands straight from L2 had a quarter of the chain, but L2 bound it at 25 B a cycle and CU (12.3 us and
-// 200 us on the same).
+// questions, whose 64-query tiles do not fill the CUs, the chain over the key blocks.  Otherwise a wave has
+// 16 of 64 queries.  SPLIT halves the chain: 32 queries per workgroup and two waves per 16; each wave
+// scores 32 keys of a block, the block's maximum and the probabilities meet in LDS, and each wave
+// multiplies them into 32 of the 64 d.  Two buffers per operand keep the next block's loads in flight
+// under this one's products, and the barrier that publishes the probabilities publishes that block too.
+// Every sum keeps its order, so both forms give the same bits.
+// Two questions of 112 and 318 tokens, 16 heads: 19.8 -> 13.5 us; one of 128 tokens 9.3 -> 6.8; 32 questions,
+// 9953 tokens (whole tiles; heads that keep to an XCD, row max and sum without LDS) 184 -> 166, sliding 84 -> 79.
+// A running maximum and sum for each half of the block's keys, joined at the end, measured 11.5 and 152 us,
+// but other sums: in fp32 a pass's logits then move by as much as they are exact to.  Keys on four waves with
+// operands straight from L2: 12.3 and 200 us, L2 binding at 25 B a cycle and CU.
 // ======================================================================================
 template <bool SPLIT>
 __global__ __launch_bounds__(256) void k_attention_f32(const float* __restrict__ Q, const float* __restrict__ K, int ldqk,
@@ -62,46 +62,45 @@ __global__ __launch_bounds__(256) void k_attention_f32(const float* __restrict__
                                                        const AttnTile* __restrict__ tiles, const int* __restrict__ soff,
                                                        const int* __restrict__ vlen, const int* __restrict__ gq,
                                                        const int* __restrict__ grow, int window_half, float scale) {
-  constexpr int NQ = SPLIT ? 32 : 64, NB = SPLIT ? 2 : 1, NC = SPLIT ? 1 : 2;
+  constexpr int NQ = SPLIT ? 32 : 64, NB = SPLIT ? 2 : 1;
+  constexpr int NP = SPLIT ? 2 : 4;                      // 16-key parts that a wave scores, 16-d parts of its output
   __shared__ f32x4_t Ks[NB][64 * 16], Vs[NB][64 * 16];
+  __shared__ f32x4_t Ps[SPLIT ? 2 : 1][SPLIT ? 4 : 1][64];  // [query group][16 keys][lane]
+  __shared__ float Ms[SPLIT ? 4 : 1][16];                // [wave][query]
 
   // heads are the fastest grid dimension: with H a multiple of 8 a head's K and V^T stay in one XCD's L2
   AttnTile tile = tiles[SPLIT ? blockIdx.y >> 1 : blockIdx.y];
   const int sub = SPLIT ? (int)(blockIdx.y & 1) * 32 : 0;
   if (sub >= tile.nq) return;                            // (also an empty tile of the pass's tile capacity)
-  tile.q0 += sub;
-  tile.nq = min(tile.nq - sub, NQ);
   const int h = blockIdx.x;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
+  const int qg = SPLIT ? wave >> 1 : wave, c0 = SPLIT ? (wave & 1) * 2 : 0;
   const int b = tile.seq, len = vlen[b], base = soff[b];
+  const bool win = window_half > 0 && !gq;
+  // the tile's blocks start here; these queries' keys: blocks that overlap [first, hi)
+  const int lo = win ? max(0, tile.q0 - window_half) & ~15 : 0;
+  tile.q0 += sub;
+  tile.nq = min(tile.nq - sub, NQ);
+  const int first = win ? max(0, tile.q0 - window_half) : 0;
+  const int hi = win ? min(len, tile.q0 + tile.nq + window_half) : len;
 
-  // this lane's query and the keys it sees, [jlo, jhi)
-  const int r = (SPLIT ? wave >> 1 : wave) * 16 + l16;
+  // this lane's query
+  const int r = qg * 16 + l16;
   const bool qvalid = r < tile.nq;
   const int rr = qvalid ? r : 0;
   int p, orow;
   if (gq) { const int gi = gq[tile.q0 + rr]; p = grow[gi] - base; orow = gi; }
   else { p = tile.q0 + rr; orow = base + p; }
-  const bool win = window_half > 0 && !gq;
-  const int jlo = win ? max(0, p - window_half) : 0, jhi = win ? min(len, p + window_half + 1) : len;
-  // keys of the tile
-  const int lo = win ? max(0, tile.q0 - window_half) : 0;
-  const int hi = win ? min(len, tile.q0 + tile.nq + window_half) : len;
 
   f32x4_t qf[4];                                         // Q[p][16 g + 4 c ..]
   const f32x4_t* qrow = reinterpret_cast<const f32x4_t*>(Q + (size_t)(base + p) * ldqk + h * 64);
 #pragma unroll
   for (int c = 0; c < 4; c++) qf[c] = qrow[4 * g + c];
 
-  struct State { f32x4_t o[4]; float mc, l; } s[NC];     // output, running max times c2, this lane's part of the sum
+  f32x4_t o[NP];
 #pragma unroll
-  for (int c = 0; c < NC; c++) {
-#pragma unroll
-    for (int db = 0; db < 4; db++) s[c].o[db] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-    s[c].mc = -INFINITY;
-    s[c].l = 0.f;
-  }
-  const float c2 = scale * 1.44269504088896340736f;
+  for (int d = 0; d < NP; d++) o[d] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  float m_run = -INFINITY, l_run = 0.f;
 
   // block k0 to registers (thread: chunk tid % 16 of rows tid / 16 + 16 it) and from there to LDS
   const int sr = tid >> 4, sc = tid & 15;
@@ -122,125 +121,104 @@ __global__ __launch_bounds__(256) void k_attention_f32(const float* __restrict__
     }
   };
 
-  // the 32 keys of class cls of the block at k0: scores, online softmax, output
-  auto half = [&](State& a, int buf, int k0, int cls) {
-    const int kc = k0 + 32 * cls;
-    if (kc >= hi || kc + 32 <= lo) return;
-    const f32x4_t *ks = &Ks[buf][32 * cls * 16], *vs = Vs[buf];
-    f32x4_t st[2];
-#pragma unroll
-    for (int n = 0; n < 2; n++) st[n] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int c = 0; c < 4; c++) {
-      f32x4_t kf[2];
-#pragma unroll
-      for (int n = 0; n < 2; n++) kf[n] = ks[(16 * n + l16) * 16 + ((4 * g + c) ^ l16)];
-#pragma unroll
-      for (int u = 0; u < 4; u++)
-#pragma unroll
-        for (int n = 0; n < 2; n++) st[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[n][u], qf[c][u], st[n], 0, 0, 0);
-    }
-    float mx = -INFINITY;
-#pragma unroll
-    for (int n = 0; n < 2; n++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const int j = kc + 16 * n + 4 * g + i;
-        const float v = j >= jlo && j < jhi ? st[n][i] : -INFINITY;
-        st[n][i] = v;
-        mx = fmaxf(mx, v);
-      }
-    const float m_new = fmaxf(a.mc, quad_rows_max(mx) * c2);
-    const float mz = m_new == -INFINITY ? 0.f : m_new;   // nothing visible yet: every exp2 below is 0
-    const float alpha = __builtin_amdgcn_exp2f(a.mc - mz);
-    a.mc = m_new;
-    float rs = 0.f;
-#pragma unroll
-    for (int n = 0; n < 2; n++)
-#pragma unroll
-      for (int i = 0; i < 4; i++) {
-        const float e = __builtin_amdgcn_exp2f(fmaf(st[n][i], c2, -mz));
-        st[n][i] = e;
-        rs += e;
-      }
-    a.l = fmaf(a.l, alpha, rs);
-#pragma unroll
-    for (int db = 0; db < 4; db++) a.o[db] *= alpha;
-#pragma unroll
-    for (int n = 0; n < 2; n++) {
-      f32x4_t vf[4];                                     // V^T[16 db + l16][keys kc + 16 n + 4 g ..]
-#pragma unroll
-      for (int db = 0; db < 4; db++) vf[db] = vs[(16 * db + l16) * 16 + ((8 * cls + 4 * n + g) ^ l16)];
-#pragma unroll
-      for (int u = 0; u < 4; u++)
-#pragma unroll
-        for (int db = 0; db < 4; db++) a.o[db] = __builtin_amdgcn_mfma_f32_16x16x4f32(vf[db][u], st[n][u], a.o[db], 0, 0, 0);
-    }
-  };
-
-  int k0 = lo & ~63;
+  int k0 = lo + ((first - lo) & ~63);
+  fetch(k0);
   if constexpr (SPLIT) {
-    fetch(k0);
     stage(0);
     if (k0 + 64 < hi) fetch(k0 + 64);
     __syncthreads();
-    for (int buf = 0; k0 < hi; k0 += 64, buf ^= 1) {
-      half(s[0], buf, k0, wave & 1);
+  }
+  for (int buf = 0; k0 < hi; k0 += 64) {
+    if constexpr (!SPLIT) {
+      stage(0);
+      __syncthreads();
+    }
+    f32x4_t st[4];                                       // part kb: keys k0 + 16 kb + 4 g ..; a wave's own are c0 .. c0 + NP - 1
+#pragma unroll
+    for (int n = 0; n < NP; n++) st[n] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int c = 0; c < 4; c++)
+#pragma unroll
+      for (int n = 0; n < NP; n++) {
+        const f32x4_t kf = Ks[buf][(16 * (c0 + n) + l16) * 16 + ((4 * g + c) ^ l16)];
+#pragma unroll
+        for (int u = 0; u < 4; u++) st[n] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf[u], qf[c][u], st[n], 0, 0, 0);
+      }
+
+    // ---- mask, online softmax ----
+    float mx = -INFINITY;
+#pragma unroll
+    for (int n = 0; n < NP; n++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        const int j = k0 + 16 * (c0 + n) + 4 * g + i;
+        const bool ok = j < len && (window_half == 0 || abs(p - j) <= window_half);
+        const float v = ok ? st[n][i] * scale : -INFINITY;
+        st[n][i] = v;
+        mx = fmaxf(mx, v);
+      }
+    mx = quad_rows_max(mx);
+    if constexpr (SPLIT) {
+      if (g == 0) Ms[wave][l16] = mx;
+      __syncthreads();
+      mx = fmaxf(mx, Ms[wave ^ 1][l16]);
+    }
+    const float m_new = fmaxf(m_run, mx);
+    const bool seen = m_new != -INFINITY;
+    const float alpha = seen ? __expf(m_run - m_new) : 1.f;
+#pragma unroll
+    for (int n = 0; n < NP; n++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) st[n][i] = !seen || st[n][i] == -INFINITY ? 0.f : __expf(st[n][i] - m_new);
+    if constexpr (SPLIT) {
+#pragma unroll
+      for (int n = 0; n < 2; n++) Ps[qg][c0 + n][lane] = st[n];
       if (k0 + 64 < hi) {
-        stage(buf ^ 1);                                  // last read before the previous barrier
+        stage(buf ^ 1);                                  // last read before the barrier above
         if (k0 + 128 < hi) fetch(k0 + 128);
       }
       __syncthreads();
+#pragma unroll
+      for (int kb = 0; kb < 4; kb++) st[kb] = Ps[qg][kb][lane];
     }
-  } else {
-    for (; k0 < hi; k0 += 64) {
-      fetch(k0);
-      stage(0);
-      __syncthreads();
-      half(s[0], 0, k0, 0);
-      half(s[NC - 1], 0, k0, 1);
+    float rs = 0.f;
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) rs += st[kb][i];
+    l_run = fmaf(l_run, alpha, quad_rows_sum(rs));
+    m_run = m_new;
+#pragma unroll
+    for (int d = 0; d < NP; d++) o[d] *= alpha;
+
+    // ---- O^T += V^T P^T ----
+#pragma unroll
+    for (int kb = 0; kb < 4; kb++)
+#pragma unroll
+      for (int d = 0; d < NP; d++) {
+        const f32x4_t va = Vs[buf][(16 * (c0 + d) + l16) * 16 + ((4 * kb + g) ^ l16)];   // keys 16 kb + 4 g ..
+#pragma unroll
+        for (int u = 0; u < 4; u++) o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[u], st[kb][u], o[d], 0, 0, 0);
+      }
+    if constexpr (SPLIT) {
+      buf ^= 1;
+    } else {
+      if (k0 + 64 < hi) fetch(k0 + 64);
       __syncthreads();
     }
   }
 
-  // the two classes together: the upper half's state into x
-  State x = s[NC - 1];
-  if constexpr (SPLIT) {
-    f32x4_t* os = Ks[0];
-    float* ml = reinterpret_cast<float*>(Vs[0]);
-    const int at = (wave >> 1) * 64 + lane;
-    if (wave & 1) {
-#pragma unroll
-      for (int db = 0; db < 4; db++) os[db * 128 + at] = s[0].o[db];
-      ml[at] = s[0].mc;
-      ml[128 + at] = s[0].l;
-    }
-    __syncthreads();
-    if (wave & 1) return;
-#pragma unroll
-    for (int db = 0; db < 4; db++) x.o[db] = os[db * 128 + at];
-    x.mc = ml[at];
-    x.l = ml[128 + at];
-  }
-  const float mj = fmaxf(s[0].mc, x.mc), mz = mj == -INFINITY ? 0.f : mj;
-  const float f0 = __builtin_amdgcn_exp2f(s[0].mc - mz), f1 = __builtin_amdgcn_exp2f(x.mc - mz);
-  const float l = quad_rows_sum(fmaf(x.l, f1, s[0].l * f0));
   if (!qvalid) return;
-  // o[db][i] = O^T[d = 16 db + 4 g + i][query]
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  // o[d][i] = O^T[16 (c0 + d) + 4 g + i][query]
+  const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
   float* orow_p = O + (size_t)orow * ldo + h * 64;
 #pragma unroll
-  for (int db = 0; db < 4; db++) {
-    f32x4_t v;
-#pragma unroll
-    for (int i = 0; i < 4; i++) v[i] = fmaf(x.o[db][i], f1, s[0].o[db][i] * f0) * inv;
-    *reinterpret_cast<f32x4_t*>(orow_p + 16 * db + 4 * g) = v;
-  }
+  for (int d = 0; d < NP; d++) *reinterpret_cast<f32x4_t*>(orow_p + 16 * (c0 + d) + 4 * g) = o[d] * inv;
 }
 
 // Workgroups of whole tiles (tiles times heads) up to which the split form runs: about one per CU.  Split
-// against whole tiles, us, 16 heads: 2 tiles 8.3 | 8.8 (both near the time of a launch), 7 tiles 11.8 | 17.7,
-// 13 tiles 13.2 | 14.9, 16 tiles of one question 49.4 | 50.5, 46 tiles 57.0 | 48.7, 173 tiles 197 | 152.
+// against whole tiles, us, 16 heads: 2 tiles 6.8 | 9.8, 7 tiles 13.5 | 20.7, 13 tiles 14.1 | 17.2, 16 tiles (one
+// question of 1024) 53.1 | 60.8, 46 tiles 64.1 | 52.2, 173 tiles 221 | 166.
 constexpr int64_t kAttnF32Split = 256;
 
 __device__ __forceinline__ uint32_t lds_addr_a(const void* p) {
