@@ -1,6 +1,6 @@
 // Attention over packed variable-length sequences for gfx950 (wave64 MFMA, fp32 online softmax).
-// Two kernels: k_attention_bf16 (the bf16 engine's, described above it) and k_attention_f32, the
-// fp32 engine's.
+// k_attention_bf16 and, for a few tiles, k_attention_narrow are the bf16 engine's kernels, k_attention_f32 the
+// fp32 engine's (each described above it).
 //
 // Masks: key j of the sequence is visible to query position p when j < len and, for sliding
 // layers, |p - j| <= window_half (inclusive, HF masking_utils.py:141-151).  Keys beyond the
@@ -402,8 +402,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4
   // exp2(s * c - m * c) with c = scale * log2(e), one FMA per score.  The running sum of the
   // probabilities is summed over exactly the bf16 values that the PV product uses, two at a time
   // (v_dot2c_f32_bf16 with (1, 1): a bf16 pair's sum added in fp32), into two partial sums per lane
-  // (even and odd pairs): lane l holds the keys 8 (l / 32) .. + 7 of each 16-key step, so a
-  // query's sum is lane l's plus lane l ^ 32's, taken once at the end.
+  // (the even and the odd 16-key steps, which is how k_attention_narrow's lanes hold them): lane l holds the keys 8 (l / 32) .. + 7 of each 16-key step, so a query's sum is lane l's
+  // plus lane l ^ 32's, taken once at the end.
   float lsum[2] = {0.f, 0.f};
   float m_run = -INFINITY;
   constexpr float kLazyLog2 = 8.f;
@@ -475,23 +475,20 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4
     // m_run, the exponent's reference, trails the running max: it moves (to every lane's max, with
     // the running output and sum rescaled) only when some valid query's max exceeds it by more
     // than 2^kLazyLog2 in probability, so probabilities stay at most 2^kLazyLog2 and most blocks
-    // skip the 48 multiplies of the rescale.  The first block has nothing to rescale.  Lanes past
-    // the tile's last query stand in for its first query and do not vote, so the points where a
-    // wave moves m_run depend on its own queries only, whatever the tile size; the stand-ins track
-    // their own max (their output is dropped).
+    // skip the 48 multiplies of the rescale.  The first block has nothing to rescale.  Each query
+    // decides for itself (the others' factor is 1), so its result depends on its own keys only, whatever
+    // the tile size and the queries of a wave.
+    const bool need = (mx - m_run) * c2 > kLazyLog2;       // (m_run = -inf: +inf, or NaN with no visible key)
     if (first) {
       m_run = mx;
-    } else if (__any(qvalid && (mx - m_run) * c2 > kLazyLog2)) {
-      // (m_run = -inf with a visible key: +inf > kLazyLog2; with none: NaN, no vote)
-      const float m_new = fmaxf(m_run, mx);
-      const float alpha = __builtin_amdgcn_exp2f(fmaf(m_run, c2, m_new == -INFINITY ? 0.f : -m_new * c2));
+    } else if (__any(need)) {
+      const float alpha = need ? __builtin_amdgcn_exp2f(fmaf(m_run, c2, -mx * c2)) : 1.f;
       lsum[0] *= alpha;
       lsum[1] *= alpha;
 #pragma unroll
       for (int db = 0; db < 2; db++) o[db] *= alpha;
-      m_run = m_new;
+      m_run = need ? mx : m_run;
     }
-    if (!qvalid) m_run = fmaxf(m_run, mx);
     // with no visible key yet (m_run = -inf) every exp2 below is exp2(-inf) = 0
     const float mc = m_run == -INFINITY ? 0.f : m_run * c2;
 #pragma unroll
@@ -533,7 +530,7 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4
 #pragma unroll
       for (int q = 0; q < 4; q++) {
         const bf16x2_t pr = {pb[2 * q], pb[2 * q + 1]};
-        lsum[q & 1] = __builtin_amdgcn_fdot2_f32_bf16(pr, one2, lsum[q & 1], false);
+        lsum[kk & 1] = __builtin_amdgcn_fdot2_f32_bf16(pr, one2, lsum[kk & 1], false);
       }
     }
   };
@@ -600,6 +597,214 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4
     }
 }
 
+// ======================================================================================
+// bf16 attention of a few tiles (v_mfma_f32_16x16x32_bf16): 16 queries per wave, NW waves per workgroup.
+//
+// What bounds a few questions is the chain of key blocks of one wave: 204 four-wave workgroups (three
+// questions of 557 to 867 tokens, 12 heads) leave a SIMD one wave, whose 64-key block takes about a
+// microsecond, its scores, softmax and products one after another and the fetch of the next block in
+// flight for no longer than that.  With 16 queries a wave has half of each (the accumulators are 16x16
+// blocks), two waves share a SIMD, and NS blocks of K and V^T are in an LDS ring with one barrier a
+// block.  Each wave reads all of a block from LDS for half the queries, which is why
+// many tiles keep k_attention_bf16 (there a CU has several workgroups, and LDS reads would bind).
+// Three questions of 557 to 867 tokens, 12 heads, every key: 15.3 -> 11.9 us; one of 128 tokens, 16 heads: 4.9 -> 3.8.
+// What binds now is a wave's own issue of about 230 instructions a block: a ring of 4 or 5 blocks and the next
+// block's scores under this block's softmax measured no faster (14.0, 13.5 us).
+//
+// The bits are those of k_attention_bf16.  Scores and outputs: an MFMA of K = 32 accumulates as two of
+// K = 16 do.  Key order: A row m of the score MFMA (t, n) is key 32 t + 8 (m / 4) + 4 n + m % 4, so that
+// lane l holds the keys 32 t + 8 (l / 16) .. + 7, the B operand of the 32-key PV step t and the eight
+// consecutive keys of a step that a lane of the other kernel sums.
+// sub: workgroups per tile (a 128-query tile as two of 64; one otherwise).
+// ======================================================================================
+template <int NW>
+__global__ __launch_bounds__(64 * NW) void k_attention_narrow(const bf16_t* __restrict__ Q, const bf16_t* __restrict__ K, int ldqk,
+                                                              int kv_rows, const bf16_t* __restrict__ Vt, int ldv, int vt_rows,
+                                                              bf16_t* __restrict__ O, int ldo, const AttnTile* __restrict__ tiles,
+                                                              int sub, const int* __restrict__ soff, const int* __restrict__ vlen,
+                                                              const int* __restrict__ gq, const int* __restrict__ grow,
+                                                              int window_half, float scale) {
+  constexpr int NS = 3, J = 8 / NW;                      // blocks in the ring; DMA instructions per wave, operand and block
+  static_assert(NW == 4 || NW == 8, "four or eight waves");
+  // [block][K rows, V^T rows][8 chunks of 16 bytes]: chunk c of row r sits at c ^ fk(r) (K) or c ^ ((r >> 1) & 7)
+  // (V^T), so that the 16 rows a fragment read touches lie in 16 different bank groups
+  __shared__ u32x4_t L[NS][2][64 * 8];
+  auto fk = [](int r) { return ((r >> 1) & 1) | (((r >> 3) & 3) << 1); };
+
+  AttnTile tile = tiles[sub == 2 ? blockIdx.y >> 1 : blockIdx.y];
+  const int off = sub == 2 ? (int)(blockIdx.y & 1) * 64 : 0;
+  if (off >= tile.nq) return;                            // (also an empty tile of the pass's tile capacity)
+  tile.q0 += off;
+  tile.nq = min(tile.nq - off, 16 * NW);
+  const int h = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
+  const int b = tile.seq, len = vlen[b], base = soff[b];
+
+  const int r = wave * 16 + l16;
+  const bool qvalid = r < tile.nq;
+  const int rr = qvalid ? r : 0;
+  int p, orow;
+  if (gq) { const int gi = gq[tile.q0 + rr]; p = grow[gi] - base; orow = gi; }
+  else { p = tile.q0 + rr; orow = base + p; }
+  const bool win = window_half > 0 && !gq;
+  const int lo = win ? max(0, tile.q0 - window_half) & ~15 : 0;
+  const int hi = win ? min(len, tile.q0 + tile.nq + window_half) : len;
+  const int jlo = win ? max(0, p - window_half) : 0, jhi = win ? min(len, p + window_half + 1) : len;
+  // keys that every query of the tile sees
+  const int jlo_all = win ? max(0, tile.q0 + tile.nq - 1 - window_half) : 0;
+  const int jhi_all = win ? min(len, tile.q0 + window_half + 1) : len;
+
+  // Q fragments: d = 32 s + 8 g .. + 7 (inline assembly, as in k_attention_bf16: the wait below defines them)
+  const char* qa = reinterpret_cast<const char*>(Q + (size_t)(base + p) * ldqk + h * 64) + 16 * g;
+  u32x4_t qf[2];
+  asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(qf[0]) : "v"(qa) : "memory");
+  asm volatile("global_load_dwordx4 %0, %1, off offset:64" : "=v"(qf[1]) : "v"(qa) : "memory");
+
+  // DMA plan: instruction j of this wave fills rows 8 i .. + 7 of the K block and of the V^T block, i = wave J + j;
+  // blocks from `hi` on come from a resource without records (zeros, no traffic), so that every block is J
+  // instructions per operand
+  const u32x4_t rK = attn_rsrc(K, (uint32_t)((size_t)kv_rows * ldqk * 2));
+  const u32x4_t rV = attn_rsrc(Vt, (uint32_t)((size_t)vt_rows * ldv * 2));
+  const uint32_t l0 = lds_addr_a(L);
+  const int wv = __builtin_amdgcn_readfirstlane(wave);
+  uint32_t kvo[J], vvo[J];
+#pragma unroll
+  for (int j = 0; j < J; j++) {
+    const int row = 8 * (wv * J + j) + (lane >> 3), c = lane & 7;
+    kvo[j] = ((uint32_t)(base + row) * (uint32_t)ldqk + (uint32_t)(h * 64)) * 2u + (uint32_t)(c ^ fk(row)) * 16u;
+    vvo[j] = ((uint32_t)(h * 64 + row) * (uint32_t)ldv + (uint32_t)base) * 2u + (uint32_t)(c ^ ((row >> 1) & 7)) * 16u;
+  }
+  auto fetch = [&](int k0, int buf) {
+    u32x4_t k = rK, v = rV;
+    if (k0 >= hi) k[2] = v[2] = 0u;
+    const uint32_t at = l0 + (uint32_t)buf * 16384u + (uint32_t)(wv * J) * 1024u;
+#pragma unroll
+    for (int j = 0; j < J; j++) {
+      attn_dma16(k, at + j * 1024u, kvo[j] + (uint32_t)k0 * (uint32_t)ldqk * 2u);
+      attn_dma16(v, at + 8192u + j * 1024u, vvo[j] + (uint32_t)k0 * 2u);
+    }
+  };
+
+  f32x4_t o[4];
+#pragma unroll
+  for (int db = 0; db < 4; db++) o[db] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+  float lsum = 0.f;
+  float m_run = -INFINITY;
+  constexpr float kLazyLog2 = 8.f;
+  const bf16x2_t one2 = {(__bf16)1.f, (__bf16)1.f};
+  const float c2 = scale * 1.44269504088896340736f;
+
+#pragma unroll
+  for (int i = 0; i < NS - 1; i++) fetch(lo + 64 * i, i);
+  asm volatile("s_waitcnt vmcnt(%2)" : "+v"(qf[0]), "+v"(qf[1]) : "n"((NS - 1) * 2 * J) : "memory");
+
+  const int krow = 8 * (l16 >> 2) + (l16 & 3);
+  int buf = 0;
+  for (int k0 = lo; k0 < hi; k0 += 64) {
+    // this block has landed (this wave's part; the barrier: all of it), and no wave still reads the block
+    // before it, whose buffer the fetch refills
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((NS - 2) * 2 * J) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    fetch(k0 + 64 * (NS - 1), buf == 0 ? NS - 1 : buf - 1);
+    const u32x4_t *ks = L[buf][0], *vs = L[buf][1];
+    buf = buf + 1 == NS ? 0 : buf + 1;
+
+    f32x4_t st[2][2];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int n = 0; n < 2; n++) {
+        st[t][n] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        const int row = 32 * t + krow + 4 * n;
+#pragma unroll
+        for (int s = 0; s < 2; s++) {
+          const u32x4_t kf = ks[row * 8 + ((4 * s + g) ^ fk(row))];
+          st[t][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, kf), __builtin_bit_cast(bf16x8_t, qf[s]),
+                                                             st[t][n], 0, 0, 0);
+        }
+      }
+    // element (t, n, i) holds key k0 + 32 t + 8 g + 4 n + i
+    if (k0 < jlo_all || k0 + 64 > jhi_all) {
+      const int A = jlo - k0 - 8 * g, B = jhi - k0 - 8 * g;
+#pragma unroll
+      for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int n = 0; n < 2; n++)
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            const int c = 32 * t + 4 * n + i;
+            st[t][n][i] = c >= A && c < B ? st[t][n][i] : -INFINITY;
+          }
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+      for (int n = 0; n < 2; n++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) mx = fmaxf(mx, st[t][n][i]);
+    mx = quad_rows_max(mx);
+    // the trailing running max of k_attention_bf16
+    const bool need = (mx - m_run) * c2 > kLazyLog2;
+    if (k0 == lo) {
+      m_run = mx;
+    } else if (__any(need)) {
+      const float alpha = need ? __builtin_amdgcn_exp2f(fmaf(m_run, c2, -mx * c2)) : 1.f;
+      lsum *= alpha;
+#pragma unroll
+      for (int db = 0; db < 4; db++) o[db] *= alpha;
+      m_run = need ? mx : m_run;
+    }
+    const float mc = m_run == -INFINITY ? 0.f : m_run * c2;
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+      bf16x8_t pb;
+#pragma unroll
+      for (int n = 0; n < 2; n++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) pb[4 * n + i] = (__bf16)__builtin_amdgcn_exp2f(fmaf(st[t][n][i], c2, -mc));
+#pragma unroll
+      for (int db = 0; db < 4; db++) {
+        const int d = 16 * db + l16;
+        const u32x4_t va = vs[d * 8 + ((4 * t + g) ^ ((d >> 1) & 7))];
+        o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, va), pb, o[db], 0, 0, 0);
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const bf16x2_t pr = {pb[2 * q], pb[2 * q + 1]};
+        lsum = __builtin_amdgcn_fdot2_f32_bf16(pr, one2, lsum, false);
+      }
+    }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");         // the fetches past the last block
+
+  // lanes l, l ^ 32 (the other 16-key steps of the same eight keys), then l ^ 16
+  const auto l2 = __builtin_amdgcn_permlane32_swap(__float_as_uint(lsum), __float_as_uint(lsum), false, false);
+  const float l3 = __uint_as_float(l2[0]) + __uint_as_float(l2[1]);
+  const auto l4 = __builtin_amdgcn_permlane16_swap(__float_as_uint(l3), __float_as_uint(l3), false, false);
+  const float l_run = __uint_as_float(l4[0]) + __uint_as_float(l4[1]);
+  if (!qvalid) return;
+  // o[db][i] = O^T[d = 16 db + 4 g + i][query]
+  const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
+  bf16_t* orow_p = O + (size_t)orow * ldo + h * 64;
+#pragma unroll
+  for (int db = 0; db < 4; db++) {
+    u32x2_t u;
+    u[0] = (uint32_t)f2bf(o[db][0] * inv) | ((uint32_t)f2bf(o[db][1] * inv) << 16);
+    u[1] = (uint32_t)f2bf(o[db][2] * inv) | ((uint32_t)f2bf(o[db][3] * inv) << 16);
+    *reinterpret_cast<u32x2_t*>(orow_p + 16 * db + 4 * g) = u;
+  }
+}
+
+// Workgroups (tiles times heads) up to which the narrow kernel runs, on 64- and on 128-query tiles, and
+// below which it takes a 128-query tile (without a window: a window's first block belongs to the tile) as
+// two.  us, k_attention_bf16 | narrow: 64-query sliding tiles, 16 heads: 2 tiles 4.6 | 4.0, 46 (736
+// workgroups, the three a CU that its LDS holds) 8.0 | 7.4, 72 10.4 | 11.5.  128-query global tiles,
+// | narrow | as two: 1 tile 5.0 | 4.6 | 3.8, 8 (1024 tokens) 16.5 | 14.9 | 11.9, 16 (256 workgroups) 17.6 | 15.6 | 16.1,
+// 25 12.7 | 12.4 | 13.2, 95 32.3 | 32.1 | 37.3, 160 55.8 | 59.7 | 67.2.
+constexpr int64_t kAttnNarrow64 = 768, kAttnNarrow128 = 512, kAttnNarrowHalves = 256;
+
 template <typename T>
 void launch_attention(const T* Q, const T* K, int ldqk, int kv_rows, const T* Vt, int ldv, T* O, int ldo,
                       const AttnTile* tiles, int ntiles, int qtile, int H, const int* soff, const int* vlen,
@@ -612,6 +817,17 @@ void launch_attention(const T* Q, const T* K, int ldqk, int kv_rows, const T* Vt
     exit(1);
   }
   if constexpr (sizeof(T) == 2) {
+    const int64_t wgs = (int64_t)ntiles * H;
+    if (wgs <= (qtile == 128 ? kAttnNarrow128 : kAttnNarrow64)) {
+      const int sub = qtile == 128 && wgs < kAttnNarrowHalves && window_half == 0 ? 2 : 1;
+      if (qtile / sub == 128)
+        LAYA_LAUNCH(k_attention_narrow<8>, dim3(H, ntiles), dim3(512), 0, st, Q, K, ldqk, kv_rows, Vt, ldv, H * 64, O, ldo, tiles,
+                    1, soff, vlen, gq, grow, window_half, scale);
+      else
+        LAYA_LAUNCH(k_attention_narrow<4>, dim3(H, ntiles * sub), dim3(256), 0, st, Q, K, ldqk, kv_rows, Vt, ldv, H * 64, O, ldo,
+                    tiles, sub, soff, vlen, gq, grow, window_half, scale);
+      return;
+    }
     if (qtile == 128)
       LAYA_LAUNCH(k_attention_bf16<4>, dim3(H, ntiles), dim3(256), 0, st, Q, K, ldqk, kv_rows, Vt, ldv, H * 64, O,
                          ldo, tiles, soff, vlen, gq, grow, window_half, scale);

@@ -289,27 +289,38 @@ def test_attention_gathered_queries(dtype):
         moff += len(m)
 
 
-@pytest.mark.parametrize("window_half", [0, 64, 7, 100])
-def test_attention_fp32_split_and_whole_tiles(window_half):
-    """The fp32 kernel's two forms: a batch whose tiles fill the CUs (whole 64-query tiles) and each of its
-    questions alone (32-query workgroups, the keys of a block on two waves) give the same bits, against
-    the fp64 oracle, with windows that are no multiple of a block too; without a window also as gathered
-    queries."""
-    pk = Packed(EDGE_LENS + [33, 31, 700, 1024], 16, "fp32", seed=15)
-    tiles = pk.encoder_tiles(64)
-    whole = pk.run(tiles, window_half)
+@pytest.mark.parametrize("dtype,qtile,window_half", [("fp32", 64, w) for w in (0, 64, 7, 100)] +
+                         [("bf16", 64, w) for w in (0, 64, 7, 100)] + [("bf16", 128, w) for w in (0, 64)])
+def test_attention_few_and_many_tiles(dtype, qtile, window_half):
+    """The forms that the number of tiles chooses between give the same bits: a batch whose tiles fill the
+    CUs, half of it, and each of its questions alone.  fp32: whole 64-query tiles against the keys of a
+    block on two waves; bf16: 32 against 16 queries per wave, and a 128-query tile as one workgroup and as
+    two.  Against the fp64 oracle too, with windows that are no multiple of a block; scores that spread
+    so wide that running maxima move often; without a window also as gathered queries."""
+    # (fp32: half as wide, because the scores' own rounding, 2^-24 of sum |q k| / 8, which is 30 and more at the
+    # bf16 scale, becomes a relative error of the probabilities and would use up the 1e-5 of _check)
+    scale = 4.0 if dtype == "bf16" else 2.0
+    pk = Packed(EDGE_LENS + [33, 31, 700, 1024], 16, dtype, seed=15, qscale=scale, kramp=scale / 2)
+    tiles = pk.encoder_tiles(qtile)
+    whole = pk.run(tiles, window_half, qtile)
     rows = [np.arange(pk.soff[b], pk.soff[b] + L) for b, L in enumerate(pk.lens)]
+    groups = [[b] for b in range(len(pk.lens))] + [list(range(0, len(pk.lens), 2)), list(range(1, len(pk.lens), 2))]
+    for group in groups:
+        part = pk.run(np.ascontiguousarray(tiles[np.isin(tiles[:, 0], group) & (tiles[:, 2] > 0)]), window_half, qtile)
+        for b in group:
+            assert np.array_equal(part[rows[b]], whole[rows[b]]), (group, b, pk.lens[b])
     for b, L in enumerate(pk.lens):
-        alone = pk.run(np.ascontiguousarray(tiles[(tiles[:, 0] == b) & (tiles[:, 2] > 0)]), window_half)
-        assert np.array_equal(alone[rows[b]], whole[rows[b]]), (b, L)
         _check(pk, whole[rows[b]], b, np.arange(L), window_half, False)
-    if window_half == 0:
+    if window_half == 0 and qtile == 64:
         grow = np.concatenate(rows).astype(np.int32)
         at = np.concatenate([[0], np.cumsum(pk.lens)])
         gt = tiles.copy()
         gt[:, 1] += at[gt[:, 0]].astype(np.int32)
-        gathered = pk.run(gt, 0, gq=np.arange(len(grow), dtype=np.int32), grow=grow, out_rows=len(grow))
-        assert np.array_equal(gathered, whole[grow])
+        ids = np.arange(len(grow), dtype=np.int32)
+        assert np.array_equal(pk.run(gt, 0, gq=ids, grow=grow, out_rows=len(grow)), whole[grow])
+        few = gt[(gt[:, 0] == len(pk.lens) - 1) & (gt[:, 2] > 0)]
+        got = pk.run(np.ascontiguousarray(few), 0, gq=ids, grow=grow, out_rows=len(grow))
+        assert np.array_equal(got[at[-2]:], whole[rows[-1]])
 
 
 def test_attention_rejects_bad_arguments():
