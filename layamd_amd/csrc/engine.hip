@@ -13,7 +13,8 @@
 //     Wo GEMM, x +=                                    k_gemm_xl<EPI_RESID>
 //     LN -> xn (next attn_norm) | final LN + type embedding into x
 //   head layer 0 (all rows), head layer 1 on the gathered marker + CLS rows, scorer, act head.
-// (bf16 names; the fp32 engine runs k_gemm and k_attention<float>.)  The GEMM tile shapes of a
+// (bf16 names; GEMMs of few rows, and the fp32 engine's, run k_gemm_small, attention of few tiles
+// k_attention_narrow, fp32 attention k_attention_f32.)  The GEMM tile shapes of a
 // pass are timed before its first run (tune_pass) and the pass is then captured in a HIP graph.
 //
 // Semantics follow the reference's Engine::run / forward_batch (src/engine.hip:396-539) and the
@@ -41,6 +42,7 @@
 #include "laya_ext.h"
 #include "model.h"
 #include "pack.h"
+#include "prefetch.h"
 
 namespace laya {
 
@@ -614,6 +616,14 @@ struct Engine : EngineIface {
   // normalising: no reduction launch, and x is read and written once instead of twice.
   static constexpr int kLatencyStages = 4;
   bool latency = false;
+  // Bf16 passes of up to kPrefetchRows rows fetch weights ahead (Prefetch) when the encoder's do not fit the
+  // memory-side cache of 256 MB, from which the next pass would read them again.  us per pass without | with:
+  // large model (686 MB) 16 rows 1249 | 1155, 128 1305 | 1220 (calls with new questions 1313 | 1253), 304 1613 | 1521,
+  // 608 1977 | 1840, 2000 3217 | 3152; base shape (218 MB) 640 rows, new questions, 1208 | 1225.  Above, the
+  // GEMMs compute for longer than their weights take.  (fp32 is bound by its MFMAs at any size: 128 rows
+  // 2334 | 2346.)  Which launch fetches which weight makes no difference.
+  static constexpr int kPrefetchRows = 2048;
+  static constexpr size_t kPrefetchBytes = (size_t)256 << 20;
   PendingPartials pend;                               // partials the next LayerNorm over all rows adds
   void splitk_latency(GemmArgs& g) {
     if (!latency || sizeof(T) != 2 || !sk_ws || g.Xh || g.K % 64) return;
@@ -805,6 +815,16 @@ struct Engine : EngineIface {
         g.Xh = xn; g.ldxh = D; g.stats = ln_stats; g.ldst = (int)MT;
       }
     };
+    const size_t encoder_bytes = (size_t)cfg.n_layers * ((size_t)4 * D * D + (size_t)3 * D * I) * sizeof(T);
+    // a pass of few rows fetches the encoder's weights ahead: Wqkv with attn_norm, Wo and Wi with the
+    // attention (a few tiles' kernel), Wmo with mlp_norm
+    auto ahead = [&](Prefetch& f, const T* w0, size_t n0, const T* w1, size_t n1) -> const Prefetch* {
+      if (sizeof(T) != 2 || T_ > kPrefetchRows || encoder_bytes <= kPrefetchBytes) return nullptr;
+      f.add(0, w0, n0 * sizeof(T));
+      f.add(1, w1, n1 * sizeof(T));
+      return &f;
+    };
+    Prefetch pf;
     for (int L = 0; L < cfg.n_layers; L++) {
       const EncLayer& e = enc[L];
       const bool glob = cfg.global_layer[L] != 0;
@@ -822,7 +842,8 @@ struct Engine : EngineIface {
       STAGE(glob ? "enc:attn_global" : "enc:attn_sliding",
             launch_attention<T>(q, k, D, (int)MT, vt, (int)VTC, ao, D, glob ? d_gltiles : d_tiles, s.nt(),
                                 glob ? lim.q_tile_global : lim.q_tile, H, d_soff, d_vlen, nullptr, nullptr,
-                                glob ? 0 : cfg.local_attention / 2, scale, st));
+                                glob ? 0 : cfg.local_attention / 2, scale, st,
+                                ahead(pf, e.Wo, (size_t)D * D, e.Wi, (size_t)2 * I * D)));
       {
         GemmArgs g = gemm_args(ao, D, e.Wo, T_, D, D, nullptr);
         g.X = x; g.ldx = D;
@@ -833,7 +854,8 @@ struct Engine : EngineIface {
       }
       if (!fold_ln)
         STAGE("enc:ln", launch_layernorm<float, T>(x, nullptr, T_, D, eps, e.mlp_norm, nullptr, nullptr, nullptr, nullptr,
-                                                   nullptr, xn, st, nullptr, take_pending()));
+                                                   nullptr, xn, st, nullptr, take_pending(),
+                                                   ahead(pf, e.Wmo, (size_t)D * I, nullptr, 0)));
       {
         GemmArgs g = gemm_args(xn, D, e.Wi, T_, 2 * I, D, nullptr);
         g.C = mg; g.ldc = I;
@@ -853,7 +875,8 @@ struct Engine : EngineIface {
       if (!last_layer) {
         if (!fold_ln)
           STAGE("enc:ln", launch_layernorm<float, T>(x, nullptr, T_, D, eps, enc[L + 1].attn_norm, nullptr, nullptr,
-                                                     nullptr, nullptr, nullptr, xn, st, nullptr, take_pending()));
+                                                     nullptr, nullptr, nullptr, xn, st, nullptr, take_pending(),
+                                                     ahead(pf, enc[L + 1].Wqkv, (size_t)3 * D * D, nullptr, 0)));
       } else {
         // final_norm then + type_emb[qtype of the row's question] (ref/rl_common.py:104), in place;
         // with the fold also its bf16 copy and statistics, which the head's first GEMM reads

@@ -8,7 +8,7 @@
 // padding rows, the next question, or the zero-initialised slack) but get probability exactly 0.
 #include <type_traits>
 
-#include "kernels.h"
+#include "prefetch.h"
 
 namespace laya {
 
@@ -615,15 +615,25 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4
 // K = 16 do.  Key order: A row m of the score MFMA (t, n) is key 32 t + 8 (m / 4) + 4 n + m % 4, so that
 // lane l holds the keys 32 t + 8 (l / 16) .. + 7, the B operand of the 32-key PV step t and the eight
 // consecutive keys of a step that a lane of the other kernel sums.
-// sub: workgroups per tile (a 128-query tile as two of 64; one otherwise).
+// sub: workgroups per tile (a 128-query tile as two of 64; one otherwise).  PF: rows of the grid from pf.ny on
+// fetch weights ahead.
 // ======================================================================================
-template <int NW>
+struct PrefetchBehind { Prefetch w; int ny; };
+template <int NW, bool PF>
 __global__ __launch_bounds__(64 * NW) void k_attention_narrow(const bf16_t* __restrict__ Q, const bf16_t* __restrict__ K, int ldqk,
                                                               int kv_rows, const bf16_t* __restrict__ Vt, int ldv, int vt_rows,
                                                               bf16_t* __restrict__ O, int ldo, const AttnTile* __restrict__ tiles,
                                                               int sub, const int* __restrict__ soff, const int* __restrict__ vlen,
                                                               const int* __restrict__ gq, const int* __restrict__ grow,
-                                                              int window_half, float scale) {
+                                                              int window_half, float scale,
+                                                              std::conditional_t<PF, PrefetchBehind, NoPrefetch> pf) {
+  if constexpr (PF) {
+    if ((int)blockIdx.y >= pf.ny) {
+      prefetch_lines(pf.w, ((blockIdx.y - pf.ny) * gridDim.x + blockIdx.x) * (64 * NW) + threadIdx.x,
+                     (gridDim.y - pf.ny) * gridDim.x * (64 * NW));
+      return;
+    }
+  }
   constexpr int NS = 3, J = 8 / NW;                      // blocks in the ring; DMA instructions per wave, operand and block
   static_assert(NW == 4 || NW == 8, "four or eight waves");
   // [block][K rows, V^T rows][8 chunks of 16 bytes]: chunk c of row r sits at c ^ fk(r) (K) or c ^ ((r >> 1) & 7)
@@ -808,7 +818,7 @@ constexpr int64_t kAttnNarrow64 = 768, kAttnNarrow128 = 512, kAttnNarrowHalves =
 template <typename T>
 void launch_attention(const T* Q, const T* K, int ldqk, int kv_rows, const T* Vt, int ldv, T* O, int ldo,
                       const AttnTile* tiles, int ntiles, int qtile, int H, const int* soff, const int* vlen,
-                      const int* gq, const int* grow, int window_half, float scale, hipStream_t st) {
+                      const int* gq, const int* grow, int window_half, float scale, hipStream_t st, const Prefetch* pf) {
   if (ntiles <= 0) return;
   // (128-query tiles give the 64-query tiles' bits only when a sliding window's half width is a
   // multiple of the 64-key block: then both tilings start their key blocks at the same keys)
@@ -820,12 +830,19 @@ void launch_attention(const T* Q, const T* K, int ldqk, int kv_rows, const T* Vt
     const int64_t wgs = (int64_t)ntiles * H;
     if (wgs <= (qtile == 128 ? kAttnNarrow128 : kAttnNarrow64)) {
       const int sub = qtile == 128 && wgs < kAttnNarrowHalves && window_half == 0 ? 2 : 1;
-      if (qtile / sub == 128)
-        LAYA_LAUNCH(k_attention_narrow<8>, dim3(H, ntiles), dim3(512), 0, st, Q, K, ldqk, kv_rows, Vt, ldv, H * 64, O, ldo, tiles,
-                    1, soff, vlen, gq, grow, window_half, scale);
-      else
-        LAYA_LAUNCH(k_attention_narrow<4>, dim3(H, ntiles * sub), dim3(256), 0, st, Q, K, ldqk, kv_rows, Vt, ldv, H * 64, O, ldo,
-                    tiles, sub, soff, vlen, gq, grow, window_half, scale);
+      const int ny = ntiles * sub;
+      auto go = [&](auto with, auto pre) {
+        constexpr bool PF = decltype(with)::value;
+        const int rows = ny + (PF ? (kPrefetchBlocks + H - 1) / H : 0);
+        if (qtile / sub == 128)
+          LAYA_LAUNCH((k_attention_narrow<8, PF>), dim3(H, rows), dim3(512), 0, st, Q, K, ldqk, kv_rows, Vt, ldv, H * 64, O, ldo,
+                      tiles, 1, soff, vlen, gq, grow, window_half, scale, pre);
+        else
+          LAYA_LAUNCH((k_attention_narrow<4, PF>), dim3(H, rows), dim3(256), 0, st, Q, K, ldqk, kv_rows, Vt, ldv, H * 64, O, ldo,
+                      tiles, sub, soff, vlen, gq, grow, window_half, scale, pre);
+      };
+      if (pf) go(std::true_type{}, PrefetchBehind{*pf, ny});
+      else go(std::false_type{}, NoPrefetch{});
       return;
     }
     if (qtile == 128)
@@ -844,6 +861,20 @@ void launch_attention(const T* Q, const T* K, int ldqk, int kv_rows, const T* Vt
   }
 }
 
+template <typename T>
+void launch_attention(const T* Q, const T* K, int ldqk, int kv_rows, const T* Vt, int ldv, T* O, int ldo,
+                      const AttnTile* tiles, int ntiles, int qtile, int H, const int* soff, const int* vlen,
+                      const int* gq, const int* grow, int window_half, float scale, hipStream_t st) {
+  launch_attention<T>(Q, K, ldqk, kv_rows, Vt, ldv, O, ldo, tiles, ntiles, qtile, H, soff, vlen, gq, grow, window_half, scale, st,
+                      nullptr);
+}
+
+template void launch_attention<float>(const float*, const float*, int, int, const float*, int, float*, int,
+                                      const AttnTile*, int, int, int, const int*, const int*, const int*, const int*,
+                                      int, float, hipStream_t, const Prefetch*);
+template void launch_attention<bf16_t>(const bf16_t*, const bf16_t*, int, int, const bf16_t*, int, bf16_t*, int,
+                                       const AttnTile*, int, int, int, const int*, const int*, const int*, const int*,
+                                       int, float, hipStream_t, const Prefetch*);
 template void launch_attention<float>(const float*, const float*, int, int, const float*, int, float*, int,
                                       const AttnTile*, int, int, int, const int*, const int*, const int*, const int*,
                                       int, float, hipStream_t);

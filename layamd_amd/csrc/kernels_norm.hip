@@ -3,7 +3,7 @@
 // LayerNorm is HBM-bound: one wave64 owns two rows (one above 1024 columns), keeps them in
 // registers (D/256 float4 per lane and row), reduces mean and variance with wave shuffles (no
 // LDS, no barriers), and writes the normalised rows in one pass.  Four waves per workgroup.
-#include "kernels.h"
+#include "prefetch.h"
 #include <type_traits>
 
 namespace laya {
@@ -35,12 +35,20 @@ template <> struct St4<bf16_t> {
 
 // Each wave normalises RPW rows; all of their loads are issued before the first reduction so
 // every lane keeps 4*RPW 16-byte loads in flight.
-template <typename Tin, typename T, int RPW, int NCH, bool MR>
+template <typename Tin, typename T, int RPW, int NCH, bool MR, bool PF>
 __global__ __launch_bounds__(256) void k_layernorm(const Tin* x, const int* __restrict__ gather, int rows, int D,
                                                    float eps, const float* __restrict__ w, const float* __restrict__ b,
                                                    const float* __restrict__ addtab, const int* __restrict__ qt,
                                                    const int* __restrict__ seq, float* y32,  // may alias x
-                                                   T* __restrict__ yT, float* __restrict__ ymr) {
+                                                   T* __restrict__ yT, float* __restrict__ ymr,
+                                                   std::conditional_t<PF, Prefetch, NoPrefetch> pf) {
+  if constexpr (PF) {
+    const int nb = (rows + 4 * RPW - 1) / (4 * RPW);    // workgroups of rows; the others prefetch
+    if ((int)blockIdx.x >= nb) {
+      prefetch_lines(pf, ((uint32_t)blockIdx.x - nb) * 256 + threadIdx.x, ((uint32_t)gridDim.x - nb) * 256);
+      return;
+    }
+  }
   const int lane = threadIdx.x & 63;
   const int row0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * RPW;
   const int nc = D >> 2;
@@ -212,7 +220,7 @@ __global__ __launch_bounds__(256) void k_layernorm_ps(const float* __restrict__ 
 template <typename Tin, typename T>
 void launch_layernorm(const Tin* x, const int* gather, int rows, int D, float eps, const float* w, const float* b,
                       const float* addtab, const int* qt, const int* seq, float* y32, T* yT, hipStream_t st,
-                      float* ymr, const PendingPartials* pend) {
+                      float* ymr, const PendingPartials* pend, const Prefetch* pf) {
   if (D % 4 || D > kLnMaxChunks * 256) {
     fprintf(stderr, "[laya] layernorm: unsupported width %d\n", D);
     exit(1);
@@ -231,21 +239,39 @@ void launch_layernorm(const Tin* x, const int* gather, int rows, int D, float ep
                   seq, y32, yT, *pend);
     return;
   }
-  auto go = [&](auto mr) {
-    constexpr bool MR = decltype(mr)::value;
+  auto go = [&](auto mr, auto with, auto pre) {
+    constexpr bool MR = decltype(mr)::value, PF = decltype(with)::value;
+    constexpr int extra = PF ? kPrefetchBlocks : 0;
     if (D <= 1024) {
       constexpr int RPW = 2;
-      LAYA_LAUNCH((k_layernorm<Tin, T, RPW, 4, MR>), dim3((rows + 4 * RPW - 1) / (4 * RPW)), dim3(256), 0, st, x,
-                         gather, rows, D, eps, w, b, addtab, qt, seq, y32, yT, ymr);
+      LAYA_LAUNCH((k_layernorm<Tin, T, RPW, 4, MR, PF>), dim3((rows + 4 * RPW - 1) / (4 * RPW) + extra), dim3(256), 0, st, x,
+                         gather, rows, D, eps, w, b, addtab, qt, seq, y32, yT, ymr, pre);
     } else {
-      LAYA_LAUNCH((k_layernorm<Tin, T, 1, kLnMaxChunks, MR>), dim3((rows + 3) / 4), dim3(256), 0, st, x, gather, rows,
-                         D, eps, w, b, addtab, qt, seq, y32, yT, ymr);
+      LAYA_LAUNCH((k_layernorm<Tin, T, 1, kLnMaxChunks, MR, PF>), dim3((rows + 3) / 4 + extra), dim3(256), 0, st, x, gather, rows,
+                         D, eps, w, b, addtab, qt, seq, y32, yT, ymr, pre);
     }
   };
-  if (ymr) go(std::true_type{});
-  else go(std::false_type{});
+  if (ymr) go(std::true_type{}, std::false_type{}, NoPrefetch{});
+  else if (pf) go(std::false_type{}, std::true_type{}, *pf);
+  else go(std::false_type{}, std::false_type{}, NoPrefetch{});
 }
 
+template <typename Tin, typename T>
+void launch_layernorm(const Tin* x, const int* gather, int rows, int D, float eps, const float* w, const float* b,
+                      const float* addtab, const int* qt, const int* seq, float* y32, T* yT, hipStream_t st,
+                      float* ymr, const PendingPartials* pend) {
+  launch_layernorm(x, gather, rows, D, eps, w, b, addtab, qt, seq, y32, yT, st, ymr, pend, nullptr);
+}
+
+template void launch_layernorm<float, float>(const float*, const int*, int, int, float, const float*, const float*,
+                                             const float*, const int*, const int*, float*, float*, hipStream_t, float*,
+                                             const PendingPartials*, const Prefetch*);
+template void launch_layernorm<float, bf16_t>(const float*, const int*, int, int, float, const float*, const float*,
+                                              const float*, const int*, const int*, float*, bf16_t*, hipStream_t, float*,
+                                              const PendingPartials*, const Prefetch*);
+template void launch_layernorm<bf16_t, bf16_t>(const bf16_t*, const int*, int, int, float, const float*, const float*,
+                                               const float*, const int*, const int*, float*, bf16_t*, hipStream_t, float*,
+                                               const PendingPartials*, const Prefetch*);
 template void launch_layernorm<float, float>(const float*, const int*, int, int, float, const float*, const float*,
                                              const float*, const int*, const int*, float*, float*, hipStream_t, float*,
                                              const PendingPartials*);
