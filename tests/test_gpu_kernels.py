@@ -4,7 +4,7 @@
     2624x1024; M = 512 and 16384; bf16 and fp32 operands, fp32 accumulate) against an fp64 CPU
     product, as the reference checks its GEMM at the layer shapes against a library
     (bench/probes/wgemm_bench.cpp:29-57);
-  * the attention kernels (bf16 k_attention_bf16, the benchmarked one, and the fp32 k_attention)
+  * the attention kernels (bf16 k_attention_bf16, the benchmarked one, and the fp32 k_attention_f32)
     in the engine's packed layout against fp64 masked softmax attention: sliding windows (+-64
     keys, inclusive, HF masking_utils.py:141-151) and global attention, lengths on both sides of
     the 64-key block and window edges, the ModernBERT-large b32 x s512 and mmBERT-base b16 x s1024
