@@ -262,6 +262,11 @@ __device__ __forceinline__ void attn_dma16(u32x4_t rsrc, uint32_t lds, uint32_t 
                : "memory");
 }
 
+// the same inside a longer asm block (offset %v, resource %r), and the step of M0 (an in-out operand of the
+// block) to the next one's base
+#define ATTN_DMA(v, r) "s_nop 0\n\tbuffer_load_dwordx4 %" v ", %" r ", 0 offen lds\n\t"
+#define ATTN_M0(bytes) "s_add_u32 m0, m0, " bytes "\n\t"
+
 __device__ __forceinline__ u32x4_t attn_rsrc(const void* p, uint32_t bytes) {
   const uint64_t v = reinterpret_cast<uint64_t>(p);
   u32x4_t r;
@@ -359,16 +364,6 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4
   const int jlo_all = win ? max(0, tile.q0 + tile.nq - 1 - window_half) : 0;
   const int jhi_all = win ? min(len, tile.q0 + window_half + 1) : len;
 
-  // Q fragments (B operand): query row, d = 16 s + 8 hi .. + 7.  Loaded by inline assembly, so
-  // that the compiler's wait analysis does not count them: the wait before the key loop below
-  // (which is also what defines qf for the compiler) lets the first V^T block stay in flight.
-  const char* qa = reinterpret_cast<const char*>(Q + (size_t)(base + p) * ldqk + h * HD) + 16 * hi;
-  u32x4_t qf[4];
-  asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(qf[0]) : "v"(qa) : "memory");
-  asm volatile("global_load_dwordx4 %0, %1, off offset:32" : "=v"(qf[1]) : "v"(qa) : "memory");
-  asm volatile("global_load_dwordx4 %0, %1, off offset:64" : "=v"(qf[2]) : "v"(qa) : "memory");
-  asm volatile("global_load_dwordx4 %0, %1, off offset:96" : "=v"(qf[3]) : "v"(qa) : "memory");
-
   // DMA plan: instruction j (0..J-1 per wave) fills the 8 rows 8 g .. + 7 of the K block and of
   // the V^T block, g = (wave & 1) + 2 (j + J (wave >> 1)); lane -> row 8 g + lane / 8, position
   // lane % 8 (global chunk position ^ swizzle).  A wave's groups g all have the parity of its
@@ -410,16 +405,33 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4
   const bf16x2_t one2 = {(__bf16)1.f, (__bf16)1.f};
   const float c2 = scale * 1.44269504088896340736f;
 
+  // Q fragments (B operand: query row, d = 16 s + 8 hi .. + 7) and the first V^T block.  One asm block
+  // issues both and waits for Q (and the first K block, issued before it; loads complete in order), so that
+  // the Q registers hold their values when the compiler first sees them.  The V^T block, the last J loads,
+  // may stay in flight: the first block waits for it before its PV step, so it lands while that block's
+  // scores and softmax run.
   fetch_k(lo, Ks0);
-  fetch_v(lo);
-  // Q and the first K block have landed (this wave's part); the first V^T block (the last J loads)
-  // may still be in flight: the first block waits for it before its PV step, so it lands while
-  // that block's scores and softmax run.  Loads complete in issue order.  The wait redefines qf,
-  // so no use of the Q registers can move above it.
-  if constexpr (J == 4)
-    asm volatile("s_waitcnt vmcnt(4)" : "+v"(qf[0]), "+v"(qf[1]), "+v"(qf[2]), "+v"(qf[3]) : : "memory");
-  else
-    asm volatile("s_waitcnt vmcnt(2)" : "+v"(qf[0]), "+v"(qf[1]), "+v"(qf[2]), "+v"(qf[3]) : : "memory");
+  const char* qa = reinterpret_cast<const char*>(Q + (size_t)(base + p) * ldqk + h * HD) + 16 * hi;
+  u32x4_t qf[4];
+  {
+    uint32_t l = lds_addr_a(Vs) + wsl;
+    const uint32_t v = vvo + (uint32_t)lo * 2u, dv = (uint32_t)ldv * 32u;
+#define ATTN_Q4                                                                          \
+  "global_load_dwordx4 %0, %5, off\n\tglobal_load_dwordx4 %1, %5, off offset:32\n\t"      \
+  "global_load_dwordx4 %2, %5, off offset:64\n\tglobal_load_dwordx4 %3, %5, off offset:96\n\t"
+    if constexpr (J == 4)
+      asm volatile(ATTN_Q4 ATTN_DMA("7", "6") ATTN_M0("2048") ATTN_DMA("8", "6") ATTN_M0("2048") ATTN_DMA("9", "6")
+                   ATTN_M0("2048") ATTN_DMA("10", "6") "s_waitcnt vmcnt(4)"
+                   : "=&v"(qf[0]), "=&v"(qf[1]), "=&v"(qf[2]), "=&v"(qf[3]), "+{m0}"(l)
+                   : "v"(qa), "s"(rV), "v"(v), "v"(v + dv), "v"(v + 2u * dv), "v"(v + 3u * dv)
+                   : "memory", "scc");
+    else
+      asm volatile(ATTN_Q4 ATTN_DMA("7", "6") ATTN_M0("2048") ATTN_DMA("8", "6") "s_waitcnt vmcnt(2)"
+                   : "=&v"(qf[0]), "=&v"(qf[1]), "=&v"(qf[2]), "=&v"(qf[3]), "+{m0}"(l)
+                   : "v"(qa), "s"(rV), "v"(v), "v"(v + dv)
+                   : "memory", "scc");
+#undef ATTN_Q4
+  }
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 
@@ -664,12 +676,6 @@ __global__ __launch_bounds__(64 * NW) void k_attention_narrow(const bf16_t* __re
   const int jlo_all = win ? max(0, tile.q0 + tile.nq - 1 - window_half) : 0;
   const int jhi_all = win ? min(len, tile.q0 + window_half + 1) : len;
 
-  // Q fragments: d = 32 s + 8 g .. + 7 (inline assembly, as in k_attention_bf16: the wait below defines them)
-  const char* qa = reinterpret_cast<const char*>(Q + (size_t)(base + p) * ldqk + h * 64) + 16 * g;
-  u32x4_t qf[2];
-  asm volatile("global_load_dwordx4 %0, %1, off" : "=v"(qf[0]) : "v"(qa) : "memory");
-  asm volatile("global_load_dwordx4 %0, %1, off offset:64" : "=v"(qf[1]) : "v"(qa) : "memory");
-
   // DMA plan: instruction j of this wave fills rows 8 i .. + 7 of the K block and of the V^T block, i = wave J + j;
   // blocks from `hi` on come from a resource without records (zeros, no traffic), so that every block is J
   // instructions per operand
@@ -704,9 +710,32 @@ __global__ __launch_bounds__(64 * NW) void k_attention_narrow(const bf16_t* __re
   const bf16x2_t one2 = {(__bf16)1.f, (__bf16)1.f};
   const float c2 = scale * 1.44269504088896340736f;
 
-#pragma unroll
-  for (int i = 0; i < NS - 1; i++) fetch(lo + 64 * i, i);
-  asm volatile("s_waitcnt vmcnt(%2)" : "+v"(qf[0]), "+v"(qf[1]) : "n"((NS - 1) * 2 * J) : "memory");
+  // The first block; then Q fragments (d = 32 s + 8 g .. + 7) and the second block in one asm block that also
+  // waits for Q, so that the Q registers hold their values when the compiler first sees them (and for the
+  // first block, which the loop waits for next; the second block's 2 J loads stay in flight).
+  static_assert(NS == 3, "two blocks before the loop");
+  fetch(lo, 0);
+  const char* qa = reinterpret_cast<const char*>(Q + (size_t)(base + p) * ldqk + h * 64) + 16 * g;
+  u32x4_t qf[2];
+  {
+    u32x4_t k = rK, v = rV;
+    if (lo + 64 >= hi) k[2] = v[2] = 0u;
+    uint32_t l = l0 + 16384u + (uint32_t)(wv * J) * 1024u;
+    const uint32_t dk = (uint32_t)(lo + 64) * (uint32_t)ldqk * 2u, dv = (uint32_t)(lo + 64) * 2u;
+#define ATTN_Q2 "global_load_dwordx4 %0, %3, off\n\tglobal_load_dwordx4 %1, %3, off offset:64\n\t"
+    if constexpr (J == 1)
+      asm volatile(ATTN_Q2 ATTN_DMA("6", "4") ATTN_M0("8192") ATTN_DMA("7", "5") "s_waitcnt vmcnt(2)"
+                   : "=&v"(qf[0]), "=&v"(qf[1]), "+{m0}"(l)
+                   : "v"(qa), "s"(k), "s"(v), "v"(kvo[0] + dk), "v"(vvo[0] + dv)
+                   : "memory", "scc");
+    else
+      asm volatile(ATTN_Q2 ATTN_DMA("6", "4") ATTN_M0("8192") ATTN_DMA("7", "5") ATTN_M0("-7168") ATTN_DMA("8", "4")
+                   ATTN_M0("8192") ATTN_DMA("9", "5") "s_waitcnt vmcnt(4)"
+                   : "=&v"(qf[0]), "=&v"(qf[1]), "+{m0}"(l)
+                   : "v"(qa), "s"(k), "s"(v), "v"(kvo[0] + dk), "v"(vvo[0] + dv), "v"(kvo[J - 1] + dk), "v"(vvo[J - 1] + dv)
+                   : "memory", "scc");
+#undef ATTN_Q2
+  }
 
   const int krow = 8 * (l16 >> 2) + (l16 & 3);
   int buf = 0;

@@ -19,6 +19,43 @@ from layamd_amd import build
 HIPCC = build.HIPCC
 
 
+needs_hipcc = pytest.mark.skipif(not (os.path.exists(HIPCC) or shutil.which(HIPCC)), reason="hipcc not available")
+
+
+def _device_asm(source, tmp_path):
+    """Device assembly of one source of the library, with the library's flags."""
+    out = tmp_path / (source + ".s")
+    flags = [f for f in build.HIP_FLAGS if f != "-fPIC"] + build.TU_FLAGS.get(source, [])
+    r = subprocess.run([HIPCC] + flags + ["--cuda-device-only", "-S", "-o", str(out), os.path.join(build.CSRC, source)],
+                       capture_output=True, text=True)
+    assert r.returncode == 0, r.stderr[-2000:]
+    return out.read_text()
+
+
+@needs_hipcc
+@pytest.mark.parametrize("source", ["kernels_attn.hip", "kernels_gemm_small.hip", "kernels_norm.hip"])
+def test_inline_assembly_waits_for_its_own_register_loads(source, tmp_path):
+    """The compiler takes the output registers of an inline assembly block as written when the block
+    ends, and may move or reuse them at once.  So a block that loads into vector registers must also
+    wait for those loads: every such load is followed in its block by an s_waitcnt vmcnt(n), n no
+    larger than the number of loads issued after it (LDS DMA writes no register and may stay in flight)."""
+    asm = _device_asm(source, tmp_path)
+    blocks = re.findall(r";;#ASMSTART\n(.*?);;#ASMEND", asm, re.S)
+    for b in blocks:
+        later, waited = 0, True                            # loads issued after the last register load; are those complete
+        for line in b.splitlines():
+            line = line.split(";")[0].strip()
+            if re.match(r"(global|buffer|flat|scratch)_load", line):
+                if not line.endswith(" lds"):
+                    later, waited = 0, False
+                else:
+                    later += 1
+            wait = re.match(r"s_waitcnt .*vmcnt\((\d+)\)", line)
+            if wait and int(wait.group(1)) <= later:
+                waited = True
+        assert waited, b
+
+
 @pytest.mark.skipif(not (os.path.exists(HIPCC) or shutil.which(HIPCC)), reason="hipcc not available")
 def test_attention_kernels_fit_their_occupancy(tmp_path):
     out = tmp_path / "attn.s"
