@@ -122,7 +122,7 @@ __global__ __launch_bounds__(256) void k_attention_f32(const float* __restrict__
   };
 
   int k0 = lo + ((first - lo) & ~63);
-  fetch(k0);
+  if (k0 < hi) fetch(k0);                                // (a question without keys has no last row to clamp to)
   if constexpr (SPLIT) {
     stage(0);
     if (k0 + 64 < hi) fetch(k0 + 64);

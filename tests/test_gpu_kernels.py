@@ -323,6 +323,23 @@ def test_attention_few_and_many_tiles(dtype, qtile, window_half):
         assert np.array_equal(got[at[-2]:], whole[rows[-1]])
 
 
+@pytest.mark.parametrize("dtype,H", [("fp32", 2), ("fp32", 64), ("bf16", 2), ("bf16", 130)])
+def test_attention_of_a_question_without_keys(dtype, H):
+    """A query tile of a question of length 0 at the very first row: no key is read (there is no row before
+    the first one), its output is 0, and the other question's is its own.  Few and many tiles (the two
+    forms of each type)."""
+    import torch
+    pk = Packed([40, 300], H, dtype, seed=16)
+    tiles = pk.encoder_tiles(64)
+    whole = pk.run(tiles, 0)
+    pk.dvlen = torch.as_tensor(np.array([0, 300], np.int32)).cuda()
+    for window_half in (0, 64):
+        got = pk.run(tiles, window_half)
+        assert np.all(got[:40] == 0.0)
+        if window_half == 0:
+            assert np.array_equal(got[pk.soff[1]:pk.soff[1] + 300], whole[pk.soff[1]:pk.soff[1] + 300])
+
+
 def test_attention_rejects_bad_arguments():
     """The hook refuses what the kernels cannot take (128-query tiles in fp32 or gathered mode,
     misaligned strides) before launching anything."""
