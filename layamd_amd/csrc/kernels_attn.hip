@@ -92,6 +92,14 @@ __global__ __launch_bounds__(256) void k_attention_f32(const float* __restrict__
   if (gq) { const int gi = gq[tile.q0 + rr]; p = grow[gi] - base; orow = gi; }
   else { p = tile.q0 + rr; orow = base + p; }
 
+  int k0 = lo + ((first - lo) & ~63);
+  if (k0 >= hi) {                                        // no key (a question without any has no row to fetch)
+    if (qvalid)
+#pragma unroll
+      for (int d = 0; d < NP; d++)
+        *reinterpret_cast<f32x4_t*>(O + (size_t)orow * ldo + h * 64 + 16 * (c0 + d) + 4 * g) = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    return;
+  }
   f32x4_t qf[4];                                         // Q[p][16 g + 4 c ..]
   const f32x4_t* qrow = reinterpret_cast<const f32x4_t*>(Q + (size_t)(base + p) * ldqk + h * 64);
 #pragma unroll
@@ -121,8 +129,7 @@ __global__ __launch_bounds__(256) void k_attention_f32(const float* __restrict__
     }
   };
 
-  int k0 = lo + ((first - lo) & ~63);
-  if (k0 < hi) fetch(k0);                                // (a question without keys has no last row to clamp to)
+  fetch(k0);
   if constexpr (SPLIT) {
     stage(0);
     if (k0 + 64 < hi) fetch(k0 + 64);
