@@ -717,29 +717,33 @@ __global__ __launch_bounds__(64 * NW) void k_attention_narrow(const bf16_t* __re
   const bf16x2_t one2 = {(__bf16)1.f, (__bf16)1.f};
   const float c2 = scale * 1.44269504088896340736f;
 
-  // The first block; then Q fragments (d = 32 s + 8 g .. + 7) and the second block in one asm block that also
-  // waits for Q, so that the Q registers hold their values when the compiler first sees them (and for the
-  // first block, which the loop waits for next; the second block's 2 J loads stay in flight).
+  // Q fragments (d = 32 s + 8 g .. + 7) and the first two blocks.  One asm block issues them, Q first, and waits
+  // for Q, so that the Q registers hold their values when the compiler first sees them (the fetches of the
+  // blocks, 4 J loads, stay in flight).
   static_assert(NS == 3, "two blocks before the loop");
-  fetch(lo, 0);
   const char* qa = reinterpret_cast<const char*>(Q + (size_t)(base + p) * ldqk + h * 64) + 16 * g;
   u32x4_t qf[2];
   {
-    u32x4_t k = rK, v = rV;
-    if (lo + 64 >= hi) k[2] = v[2] = 0u;
-    uint32_t l = l0 + 16384u + (uint32_t)(wv * J) * 1024u;
-    const uint32_t dk = (uint32_t)(lo + 64) * (uint32_t)ldqk * 2u, dv = (uint32_t)(lo + 64) * 2u;
+    u32x4_t k1 = rK, v1 = rV;
+    if (lo + 64 >= hi) k1[2] = v1[2] = 0u;
+    uint32_t l = l0 + (uint32_t)(wv * J) * 1024u;
+    const uint32_t dk = (uint32_t)lo * (uint32_t)ldqk * 2u, dv = (uint32_t)lo * 2u, nk = (uint32_t)ldqk * 128u;
 #define ATTN_Q2 "global_load_dwordx4 %0, %3, off\n\tglobal_load_dwordx4 %1, %3, off offset:64\n\t"
     if constexpr (J == 1)
-      asm volatile(ATTN_Q2 ATTN_DMA("6", "4") ATTN_M0("8192") ATTN_DMA("7", "5") "s_waitcnt vmcnt(2)"
+      asm volatile(ATTN_Q2 ATTN_DMA("8", "4") ATTN_M0("8192") ATTN_DMA("9", "5") ATTN_M0("8192") ATTN_DMA("10", "6")
+                   ATTN_M0("8192") ATTN_DMA("11", "7") "s_waitcnt vmcnt(4)"
                    : "=&v"(qf[0]), "=&v"(qf[1]), "+{m0}"(l)
-                   : "v"(qa), "s"(k), "s"(v), "v"(kvo[0] + dk), "v"(vvo[0] + dv)
+                   : "v"(qa), "s"(rK), "s"(rV), "s"(k1), "s"(v1), "v"(kvo[0] + dk), "v"(vvo[0] + dv), "v"(kvo[0] + dk + nk),
+                     "v"(vvo[0] + dv + 128u)
                    : "memory", "scc");
     else
-      asm volatile(ATTN_Q2 ATTN_DMA("6", "4") ATTN_M0("8192") ATTN_DMA("7", "5") ATTN_M0("-7168") ATTN_DMA("8", "4")
-                   ATTN_M0("8192") ATTN_DMA("9", "5") "s_waitcnt vmcnt(4)"
+      asm volatile(ATTN_Q2 ATTN_DMA("8", "4") ATTN_M0("8192") ATTN_DMA("9", "5") ATTN_M0("-7168") ATTN_DMA("10", "4")
+                   ATTN_M0("8192") ATTN_DMA("11", "5") ATTN_M0("7168") ATTN_DMA("12", "6") ATTN_M0("8192") ATTN_DMA("13", "7")
+                   ATTN_M0("-7168") ATTN_DMA("14", "6") ATTN_M0("8192") ATTN_DMA("15", "7") "s_waitcnt vmcnt(8)"
                    : "=&v"(qf[0]), "=&v"(qf[1]), "+{m0}"(l)
-                   : "v"(qa), "s"(k), "s"(v), "v"(kvo[0] + dk), "v"(vvo[0] + dv), "v"(kvo[J - 1] + dk), "v"(vvo[J - 1] + dv)
+                   : "v"(qa), "s"(rK), "s"(rV), "s"(k1), "s"(v1), "v"(kvo[0] + dk), "v"(vvo[0] + dv), "v"(kvo[J - 1] + dk),
+                     "v"(vvo[J - 1] + dv), "v"(kvo[0] + dk + nk), "v"(vvo[0] + dv + 128u), "v"(kvo[J - 1] + dk + nk),
+                     "v"(vvo[J - 1] + dv + 128u)
                    : "memory", "scc");
 #undef ATTN_Q2
   }
