@@ -843,7 +843,8 @@ struct Engine : EngineIface {
             launch_attention<T>(q, k, D, (int)MT, vt, (int)VTC, ao, D, glob ? d_gltiles : d_tiles, s.nt(),
                                 glob ? lim.q_tile_global : lim.q_tile, H, d_soff, d_vlen, nullptr, nullptr,
                                 glob ? 0 : cfg.local_attention / 2, scale, st,
-                                ahead(pf, e.Wo, (size_t)D * D, e.Wi, (size_t)2 * I * D)));
+                                ahead(pf, e.Wo, (size_t)D * D, e.Wi, (size_t)2 * I * D),
+                                tiles_expected(T_, B, glob ? lim.q_tile_global : lim.q_tile)));
       {
         GemmArgs g = gemm_args(ao, D, e.Wo, T_, D, D, nullptr);
         g.X = x; g.ldx = D;
@@ -903,7 +904,8 @@ struct Engine : EngineIface {
       }
       if (!last) {
         STAGE("head:attn", launch_attention<T>(q, k, D, (int)MT, vt, (int)VTC, ao, D, d_gltiles, s.nt(), lim.q_tile_global, H, d_soff,
-                                               d_vlen, nullptr, nullptr, 0, scale, st));
+                                               d_vlen, nullptr, nullptr, 0, scale, st, nullptr,
+                                               tiles_expected(T_, B, lim.q_tile_global)));
         { GemmArgs g = gemm_args(ao, D, hl.outW, T_, D, D, hl.outB); g.X = x; g.ldx = D;
           if (fold_ln) fold_out(g);
           splitk_latency(g);
@@ -924,7 +926,8 @@ struct Engine : EngineIface {
       } else {
         // queries, out-proj and FFN only for the R = KT + B rows read afterwards
         STAGE("head:attn_gathered", launch_attention<T>(q, k, D, (int)MT, vt, (int)VTC, aog, D, d_gtiles, s.ngt(), kQTile, H, d_soff,
-                                                        d_vlen, d_gq, d_grow, 0, scale, st));
+                                                        d_vlen, d_gq, d_grow, 0, scale, st, nullptr,
+                                                        tiles_expected(KT, B, kQTile)));
         STAGE("head:gather", launch_gather_rows(x, d_grow, xg, R, D, st));
         { GemmArgs g = gemm_args(aog, D, hl.outW, R, D, D, hl.outB); g.X = xg; g.ldx = D; splitk(g);
           GSTAGE("head:gemm_out_res", gemm(EPI_RESID, g, st)); }

@@ -4,6 +4,7 @@
 #include <string>
 #include <vector>
 
+#include "attn_form.h"
 #include "model.h"
 #include "pack.h"
 
@@ -55,6 +56,13 @@ int laya_host_plan(int B, const int* lens, const int* ids, const int* nmark, con
     if (grow) memcpy(grow, p.grow.data(), p.R * 4);
   }
   return (int)ps.size();
+}
+
+// The attention form (AttnForm) of a pass bucket's launch on query tiles of q_tile: rows (or, for a gathered
+// list, marker rows) and questions of the bucket; *expect gets the tiles it is chosen by.
+int laya_host_attention_form(int bf16, int rows, int B, int q_tile, int H, int window_half, int* expect) {
+  *expect = tiles_expected(rows, B, q_tile);
+  return attention_form(bf16 != 0, *expect, H, q_tile, window_half);
 }
 
 // Parses <dir>'s configs.  out[16] = n_layers, d, n_heads, head_dim, intermediate, vocab, max_len,

@@ -6,8 +6,10 @@
 // layers, |p - j| <= window_half (inclusive, HF masking_utils.py:141-151).  Keys beyond the
 // sequence are read (V^T columns up to the next 64-key boundary exist and hold finite values:
 // padding rows, the next question, or the zero-initialised slack) but get probability exactly 0.
+#include <algorithm>
 #include <type_traits>
 
+#include "attn_form.h"
 #include "prefetch.h"
 
 namespace laya {
@@ -222,11 +224,6 @@ __global__ __launch_bounds__(256) void k_attention_f32(const float* __restrict__
 #pragma unroll
   for (int d = 0; d < NP; d++) *reinterpret_cast<f32x4_t*>(orow_p + 16 * (c0 + d) + 4 * g) = o[d] * inv;
 }
-
-// Workgroups of whole tiles (tiles times heads) up to which the split form runs: about one per CU.  Split
-// against whole tiles, us, 16 heads: 2 tiles 6.8 | 9.8, 7 tiles 13.5 | 20.7, 13 tiles 14.1 | 17.2, 16 tiles (one
-// question of 1024) 53.1 | 60.8, 46 tiles 64.1 | 52.2, 173 tiles 221 | 166.
-constexpr int64_t kAttnF32Split = 256;
 
 __device__ __forceinline__ uint32_t lds_addr_a(const void* p) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)p;
@@ -847,18 +844,11 @@ __global__ __launch_bounds__(64 * NW) void k_attention_narrow(const bf16_t* __re
   }
 }
 
-// Workgroups (tiles times heads) up to which the narrow kernel runs, on 64- and on 128-query tiles, and
-// below which it takes a 128-query tile (without a window: a window's first block belongs to the tile) as
-// two.  us, k_attention_bf16 | narrow: 64-query sliding tiles, 16 heads: 2 tiles 4.6 | 4.0, 46 (736
-// workgroups, the three a CU that its LDS holds) 8.0 | 7.4, 72 10.4 | 11.5.  128-query global tiles,
-// | narrow | as two: 1 tile 5.0 | 4.6 | 3.8, 8 (1024 tokens) 16.5 | 14.9 | 11.9, 16 (256 workgroups) 17.6 | 15.6 | 16.1,
-// 25 12.7 | 12.4 | 13.2, 95 32.3 | 32.1 | 37.3, 160 55.8 | 59.7 | 67.2.
-constexpr int64_t kAttnNarrow64 = 768, kAttnNarrow128 = 512, kAttnNarrowHalves = 256;
-
 template <typename T>
 void launch_attention(const T* Q, const T* K, int ldqk, int kv_rows, const T* Vt, int ldv, T* O, int ldo,
                       const AttnTile* tiles, int ntiles, int qtile, int H, const int* soff, const int* vlen,
-                      const int* gq, const int* grow, int window_half, float scale, hipStream_t st, const Prefetch* pf) {
+                      const int* gq, const int* grow, int window_half, float scale, hipStream_t st, const Prefetch* pf,
+                      int expect) {
   if (ntiles <= 0) return;
   // (128-query tiles give the 64-query tiles' bits only when a sliding window's half width is a
   // multiple of the 64-key block: then both tilings start their key blocks at the same keys)
@@ -866,10 +856,10 @@ void launch_attention(const T* Q, const T* K, int ldqk, int kv_rows, const T* Vt
     fprintf(stderr, "[laya] attention: unsupported query tile %d (window half %d)\n", qtile, window_half);
     exit(1);
   }
+  const AttnForm form = attention_form(sizeof(T) == 2, expect > 0 ? std::min(expect, ntiles) : ntiles, H, qtile, window_half);
   if constexpr (sizeof(T) == 2) {
-    const int64_t wgs = (int64_t)ntiles * H;
-    if (wgs <= (qtile == 128 ? kAttnNarrow128 : kAttnNarrow64)) {
-      const int sub = qtile == 128 && wgs < kAttnNarrowHalves && window_half == 0 ? 2 : 1;
+    if (form != kAttnWide) {
+      const int sub = form == kAttnHalves ? 2 : 1;
       const int ny = ntiles * sub;
       auto go = [&](auto with, auto pre) {
         constexpr bool PF = decltype(with)::value;
@@ -892,7 +882,7 @@ void launch_attention(const T* Q, const T* K, int ldqk, int kv_rows, const T* Vt
       LAYA_LAUNCH(k_attention_bf16<2>, dim3(H, ntiles), dim3(128), 0, st, Q, K, ldqk, kv_rows, Vt, ldv, H * 64, O,
                          ldo, tiles, soff, vlen, gq, grow, window_half, scale);
   } else {
-    if ((int64_t)ntiles * H <= kAttnF32Split)
+    if (form == kAttnSplit)
       LAYA_LAUNCH(k_attention_f32<true>, dim3(H, ntiles * 2), dim3(256), 0, st, Q, K, ldqk, Vt, ldv, O, ldo, tiles, soff, vlen,
                   gq, grow, window_half, scale);
     else
@@ -906,15 +896,15 @@ void launch_attention(const T* Q, const T* K, int ldqk, int kv_rows, const T* Vt
                       const AttnTile* tiles, int ntiles, int qtile, int H, const int* soff, const int* vlen,
                       const int* gq, const int* grow, int window_half, float scale, hipStream_t st) {
   launch_attention<T>(Q, K, ldqk, kv_rows, Vt, ldv, O, ldo, tiles, ntiles, qtile, H, soff, vlen, gq, grow, window_half, scale, st,
-                      nullptr);
+                      nullptr, 0);
 }
 
 template void launch_attention<float>(const float*, const float*, int, int, const float*, int, float*, int,
                                       const AttnTile*, int, int, int, const int*, const int*, const int*, const int*,
-                                      int, float, hipStream_t, const Prefetch*);
+                                      int, float, hipStream_t, const Prefetch*, int);
 template void launch_attention<bf16_t>(const bf16_t*, const bf16_t*, int, int, const bf16_t*, int, bf16_t*, int,
                                        const AttnTile*, int, int, int, const int*, const int*, const int*, const int*,
-                                       int, float, hipStream_t, const Prefetch*);
+                                       int, float, hipStream_t, const Prefetch*, int);
 template void launch_attention<float>(const float*, const float*, int, int, const float*, int, float*, int,
                                       const AttnTile*, int, int, int, const int*, const int*, const int*, const int*,
                                       int, float, hipStream_t);

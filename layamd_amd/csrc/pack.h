@@ -40,6 +40,14 @@ constexpr int kMarkerBucket = 64;    // a pass's marker rows (KT) are a multiple
 // + B for q_tile >= 64, and sum of ceil((nmark + 1) / 64) <= R / 64 + B
 inline int tiles_cap(int rows, int B) { return rows / kRowBucket + B; }
 inline int gtiles_cap(int R, int B) { return R / kQTile + B; }
+// Non-empty tiles that a list of a pass bucket is expected to hold, from the bucket alone so that every batch
+// of it launches the same kernels: each question's last tile is half full on average, and each has one.
+// Exact for one question, and for questions of up to q_tile tokens when they are half of that or shorter.
+// Gathered lists: rows = KT.
+inline int tiles_expected(int rows, int B, int q_tile) {
+  const int n = (rows + q_tile - 1) / q_tile + (B - 1) / 2;
+  return n > B ? n : B;
+}
 
 struct PackLimits {
   int max_len = 512;

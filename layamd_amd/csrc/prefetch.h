@@ -31,7 +31,9 @@ __device__ __forceinline__ void prefetch_lines(const Prefetch& f, uint32_t threa
 }
 
 // launch_layernorm and launch_attention with weights to fetch ahead (null: none).  Only k_layernorm (without
-// ymr) and the bf16 attention of a few tiles add the workgroups; the other kernels ignore pf.
+// ymr) and the bf16 attention of a few tiles add the workgroups; the other kernels ignore pf.  expect: how
+// many of the ntiles tiles are not empty, as far as the caller can say (tiles_expected; 0: all), which
+// chooses the kernel (attn_form.h) and nothing else.
 template <typename Tin, typename T>
 void launch_layernorm(const Tin* x, const int* gather, int rows, int D, float eps, const float* w, const float* b,
                       const float* addtab, const int* qt, const int* seq, float* y32, T* yT, hipStream_t st, float* ymr,
@@ -39,6 +41,7 @@ void launch_layernorm(const Tin* x, const int* gather, int rows, int D, float ep
 template <typename T>
 void launch_attention(const T* Q, const T* K, int ldqk, int kv_rows, const T* Vt, int ldv, T* O, int ldo,
                       const AttnTile* tiles, int ntiles, int qtile, int H, const int* soff, const int* vlen,
-                      const int* gq, const int* grow, int window_half, float scale, hipStream_t st, const Prefetch* pf);
+                      const int* gq, const int* grow, int window_half, float scale, hipStream_t st, const Prefetch* pf,
+                      int expect);
 
 }  // namespace laya

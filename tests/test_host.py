@@ -189,6 +189,59 @@ def test_layout_properties_of_random_batches(host, data):
     assert nxt == n
 
 
+WIDE, NARROW, HALVES, SPLIT = range(4)                    # AttnForm
+
+
+def attention_form(host, bf16, p, H, q_tile, window_half, gathered=False):
+    n = ctypes.c_int()
+    f = host.laya_host_attention_form(bf16, int(p["KT"] if gathered else p["T"]), int(p["B"]), q_tile, H, window_half,
+                                      ctypes.byref(n))
+    return f, n.value
+
+
+def real(tiles):
+    return int((tiles[:, 2] > 0).sum())
+
+
+@pytest.mark.parametrize("bf16,H,lens,q_tile,window_half,form", [
+    (1, 16, [128], 64, 64, NARROW), (1, 16, [128], 128, 0, HALVES),
+    (1, 16, [1024], 128, 0, HALVES), (1, 12, [557, 640, 867], 128, 0, HALVES), (1, 16, [700, 650, 600], 128, 0, NARROW),
+    (1, 16, [1024, 1020], 128, 0, NARROW), (1, 16, [20] * 64, 64, 64, WIDE), (1, 16, [20] * 64, 128, 0, WIDE),
+    (1, 16, [311] * 32, 64, 64, WIDE), (1, 16, [311] * 32, 128, 0, WIDE),
+    (0, 16, [1024], 64, 0, SPLIT), (0, 16, [112, 318], 64, 64, SPLIT), (0, 12, [1024], 64, 0, SPLIT),
+    (0, 16, [1024, 64], 64, 0, WIDE), (0, 12, [1024, 400], 64, 0, WIDE)])
+def test_attention_form_of_a_pass(host, bf16, H, lens, q_tile, window_half, form):
+    """A pass runs the form that the rule was measured for at its real tiles: its lists are padded to the
+    bucket's capacity, by half as many tiles again and more in the 128-query list."""
+    b = wl.make_batch(ck.PRESETS["large1024"], lens, [4] * len(lens), seed=3)
+    (p,) = plan(host, *b.flat(), max_len=1024, q_tile=64, q_tile_global=128 if bf16 else 64)
+    key = "gltiles" if window_half == 0 else "tiles"
+    got, expect = attention_form(host, bf16, p, H, q_tile, window_half)
+    assert got == form
+    assert abs(expect - real(p[key])) <= len(lens) // 2 + 1
+
+
+@settings(max_examples=80, deadline=None, suppress_health_check=[HealthCheck.function_scoped_fixture])
+@given(data=st.data())
+def test_expected_attention_tiles_of_random_batches(host, data):
+    """One question: exactly its tiles, of either size, for every length.  Several: within what questions
+    whose last tiles are all full, or hold one query, differ from half full ones; never fewer than one each."""
+    n = data.draw(st.integers(1, 24), label="questions")
+    lens = data.draw(st.lists(st.integers(1, 1024), min_size=n, max_size=n), label="lens")
+    nm = data.draw(st.lists(st.integers(1, 255), min_size=n, max_size=n), label="markers")
+    b = wl.make_batch(ck.PRESETS["large1024"], lens, nm, seed=1)
+    (p,) = plan(host, *b.flat(), max_len=1024, q_tile=64, q_tile_global=128)
+    for key, q, rows, gathered in (("tiles", 64, p["T"], False), ("gltiles", 128, p["T"], False), ("gtiles", 64, p["KT"], True)):
+        expect = attention_form(host, 1, p, 16, q, 0, gathered)[1]
+        assert n <= expect <= len(p[key])
+        # each question's tiles are at least len / q and less than len / q + 1; a pass's rows hold at most 7 padding
+        # rows a question and 63 at its end, KT 63, and a gathered list one CLS query a question
+        slack = (7 * n + 63) / q if not gathered else (n + 63) / q
+        assert abs(expect - real(p[key])) <= n / 2 + 1 + slack
+        if n == 1 and not gathered:
+            assert expect == real(p[key])
+
+
 def test_pass_splitting(host):
     cfg = ck.PRESETS["tiny"]
     lens = [300, 200, 150, 10, 320, 64, 5]
