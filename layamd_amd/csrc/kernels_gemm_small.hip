@@ -100,7 +100,7 @@ __global__ __launch_bounds__(64 * WM * WN) void k_gemm_small(const GemmArgs a, i
   constexpr int SC = (BM + BN) * 8, SB = SC * 16;         // a stage in chunks and in bytes
   static_assert(KU == 1 || KU == 2, "stages per step");
   static_assert((BM + BN) % (8 * NW) == 0 && BM % (16 * WM) == 0 && BN % (16 * WN) == 0, "tile");
-  static_assert((NB - 2) * KU * NI <= 63 && NB >= 3, "vmcnt");
+  static_assert((NB - 1) * KU * NI <= 63 && NB >= 3, "vmcnt");
   static_assert(NB * KU * SB <= 160 * 1024, "LDS");
   constexpr int LDC = EPI == EPI_QKV ? (BN > BM ? BN : BM) + 4 : BN + 4;   // row stride of the staged tile (floats)
   static_assert((EPI == EPI_QKV && BM > BN ? BM : BM > BN ? BM : BN) * LDC * 4 <= NB * KU * SB, "staged tile");
@@ -410,25 +410,30 @@ static void launch_small(int epi, const GemmArgs& a, hipStream_t st) {
   const dim3 grid((unsigned)(((a.M + BM - 1) / BM) * ((a.N + BN - 1) / BN))), block(64 * WM * WN);
   int per = 0;
   if (a.ksplit > 1) { const int stages = a.K / 64; per = (stages + a.ksplit - 1) / a.ksplit; }
+#define LAYA_SMALL(EPI, SPLIT)                                                                          \
+  {                                                                                                     \
+    LAYA_LAUNCH((k_gemm_small<T, BM, BN, WM, WN, KU, NB, EPI, SPLIT>), grid, block, 0, st, a, per); \
+    return;                                                                                             \
+  }
   switch (epi) {
     case EPI_STORE:
-      if constexpr (sizeof(T) == 2)
-        if (per) { LAYA_LAUNCH((k_gemm_small<T, BM, BN, WM, WN, KU, NB, EPI_STORE, true>), grid, block, 0, st, a, per); return; }
-      LAYA_LAUNCH((k_gemm_small<T, BM, BN, WM, WN, KU, NB, EPI_STORE, false>), grid, block, 0, st, a, per);
-      return;
+      if constexpr (sizeof(T) == 2) if (per) LAYA_SMALL(EPI_STORE, true)
+      if constexpr (BM < 128) LAYA_SMALL(EPI_STORE, false)
+      break;
     case EPI_RESID:
-      if constexpr (sizeof(T) == 2)
-        if (per) { LAYA_LAUNCH((k_gemm_small<T, BM, BN, WM, WN, KU, NB, EPI_RESID, true>), grid, block, 0, st, a, per); return; }
-      LAYA_LAUNCH((k_gemm_small<T, BM, BN, WM, WN, KU, NB, EPI_RESID, false>), grid, block, 0, st, a, per);
-      return;
+      if constexpr (sizeof(T) == 2) if (per) LAYA_SMALL(EPI_RESID, true)
+      if constexpr (BM < 128) LAYA_SMALL(EPI_RESID, false)
+      break;
     case EPI_QKV:
-      if constexpr (BN % 64 == 0) LAYA_LAUNCH((k_gemm_small<T, BM, BN, WM, WN, KU, NB, EPI_QKV, false>), grid, block, 0, st, a, per);
-      return;
+      if constexpr (BN % 64 == 0) LAYA_SMALL(EPI_QKV, false)
+      break;
     case EPI_GEGLU:
-      if constexpr (BN % 64 == 0) LAYA_LAUNCH((k_gemm_small<T, BM, BN, WM, WN, KU, NB, EPI_GEGLU, false>), grid, block, 0, st, a, per);
-      return;
-    default: fprintf(stderr, "[laya] gemm: bad epilogue %d\n", epi); exit(1);
+      if constexpr (BN % 64 == 0 && BM < 128) LAYA_SMALL(EPI_GEGLU, false)
+      break;
   }
+#undef LAYA_SMALL
+  fprintf(stderr, "[laya] gemm: epilogue %d is not built for %dx%d tiles\n", epi, BM, BN);
+  exit(1);
 }
 
 template <typename T>
@@ -461,21 +466,23 @@ template <typename T>
 bool gemm_small_fits(int epi, const GemmArgs& a, int v) {
   const char* why = "";
   if (v < 0 || v >= kSmallVariants || !gemm_shape_ok(epi, a, (int)sizeof(T), &why)) return false;
-  if (sizeof(T) == 4 && v == 4) return false;
+  if (v == 4 && (sizeof(T) == 4 || (epi != EPI_QKV && a.ksplit <= 1))) return false;   // (the only forms it is built in)
   if (a.ln_mr || a.stats || a.Xh || a.partials_only) return false;
   auto al16 = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
   const int bn = small_tile(v).bn;
-  constexpr int e4 = 4;                                    // outputs leave in groups of four
+  // outputs leave in groups of four; bf16 ones in whole groups of 8, like those of the large tiles (the generic
+  // kernel, which takes the others, evaluates GELU in another form)
+  constexpr int eo = sizeof(T) == 2 ? 8 : 4;
   if (a.N % 8 || !al16(a.bias)) return false;
   if ((size_t)a.M * a.lda * sizeof(T) >= (1u << 31) - 65536 || (size_t)a.N * a.ldw * sizeof(T) >= (1u << 31) - 65536) return false;
   switch (epi) {
-    case EPI_STORE: if (a.ldc % e4 || !al16(a.C)) return false; break;
-    case EPI_RESID: if (a.ldx % e4 || !al16(a.X)) return false; break;
+    case EPI_STORE: if (a.ldc % eo || !al16(a.C)) return false; break;
+    case EPI_RESID: if (a.ldx % 4 || !al16(a.X)) return false; break;
     case EPI_QKV:
       if (a.HD != 64 || bn % 64 || a.H * a.HD % bn || a.ldqk % 8 || a.ldv % 8 || !al16(a.Q) || !al16(a.Kt) || !al16(a.Vt) ||
           !al16(a.rope_cos) || !al16(a.rope_sin)) return false;
       break;
-    case EPI_GEGLU: if (bn % 64 || a.ldc % e4 || !al16(a.C)) return false; break;
+    case EPI_GEGLU: if (bn % 64 || a.ldc % eo || !al16(a.C)) return false; break;
     default: return false;
   }
   if (a.ksplit > 1 && (sizeof(T) != 2 || a.ws == nullptr || (epi != EPI_STORE && epi != EPI_RESID) || a.K % 64 || a.K < 128)) return false;
@@ -537,7 +544,6 @@ int gemm_small_pick(int epi, const GemmArgs& a) {
     const SmallTile t = small_tile(v);
     const int64_t tiles = (int64_t)((a.M + t.bm - 1) / t.bm) * ((a.N + t.bn - 1) / t.bn);
     const bool split = a.ksplit > 1;
-    if (v == 4 && epi != EPI_QKV && !split) return -1;
     if ((tiles <= cus || (v == 4 && split)) && gemm_small_fits<T>(epi, a, v)) return v;
   }
   return -1;
