@@ -1093,6 +1093,7 @@ int laya_ext_prof_sequence(void* h, int* stages, int cap) {
 static float* g_ext_ws = nullptr;          // split-K workspace of laya_ext_gemm (caller's memory)
 static size_t g_ext_ws_bytes = 0;
 static int g_ext_ks = 0;                   // split-K factor pinned with it
+static int g_ext_small = -1;               // few-row variant pinned by laya_ext_gemm_small (-1: none)
 
 // The measurement hooks run inside the caller's process, which shares the HIP runtime (and its
 // per-thread last error) with the caller: a stale error that the caller's own HIP calls left must
@@ -1141,11 +1142,18 @@ int laya_ext_gemm(int dtype, int epi, const void* A, const void* W, void* C, con
   // a pinned split-K factor runs in the caller's workspace (laya_ext_gemm_ksplit)
   g.ws = g_ext_ws;
   g.ws_bytes = g_ext_ws_bytes;
+  const int e = epi == 0 ? EPI_STORE : EPI_RESID, small = g_ext_small;
+  if (small >= 0) {
+    if (dtype == 1 && g_ext_ks > 1) g.ksplit = g_ext_ks;
+    if (!(dtype == 0 ? gemm_small_fits<float>(e, g, small) : gemm_small_fits<bf16_t>(e, g, small))) return -1;
+  }
   hipEvent_t a, b;
   if (ms) { LAYA_HIP(hipEventCreate(&a)); LAYA_HIP(hipEventCreate(&b)); LAYA_HIP(hipEventRecord(a, st)); }
   for (int i = 0; i < iters; i++) {
-    const int e = epi == 0 ? EPI_STORE : EPI_RESID;
-    if (dtype == 0) {
+    if (small >= 0) {
+      if (dtype == 0) launch_gemm_small_variant<float>(e, g, small, st);
+      else launch_gemm_small_variant<bf16_t>(e, g, small, st);
+    } else if (dtype == 0) {
       if (!launch_gemm_small<float>(e, g, st)) launch_gemm<float>(e, g, st);
     } else if (g_ext_ks > 1 || !launch_gemm_small<bf16_t>(e, g, st)) {
       launch_gemm<bf16_t>(e, g, st);
@@ -1159,6 +1167,22 @@ int laya_ext_gemm(int dtype, int epi, const void* A, const void* W, void* C, con
   }
   LAYA_HIP(hipGetLastError());
   return 0;
+}
+int laya_ext_gemm_small(int variant) {
+  if (variant < -1 || variant >= laya::kSmallVariants) return -2;
+  const int prev = g_ext_small;
+  g_ext_small = variant;
+  return prev;
+}
+int laya_ext_gemm_small_pick(int dtype, int epi, int M, int N, int K, int ksplit) {
+  using namespace laya;
+  if ((dtype != 0 && dtype != 1) || (epi != 0 && epi != 1)) return -1;
+  GemmArgs g;                              // (null operands: aligned ones)
+  g.lda = K; g.ldw = K; g.M = M; g.N = N; g.K = K; g.ldc = N; g.ldx = N;
+  float ws;
+  if (ksplit > 1) { g.ksplit = ksplit; g.ws = &ws; }
+  const int e = epi == 0 ? EPI_STORE : EPI_RESID;
+  return dtype == 0 ? gemm_small_pick<float>(e, g) : gemm_small_pick<bf16_t>(e, g);
 }
 const char* laya_ext_precision(void* h) { return E(h)->precision(); }
 

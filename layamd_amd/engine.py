@@ -27,7 +27,7 @@ ABI_SYMBOLS = ["laya_create", "laya_forward_batch", "laya_forward", "laya_n_act"
 EXT_SYMBOLS = ["laya_ext_prof_enable", "laya_ext_prof_stage", "laya_ext_replay", "laya_ext_precision", "laya_ext_gemm",
                "laya_ext_gemm_config", "laya_ext_gemm_split", "laya_ext_gemm_ksplit", "laya_ext_mfma_loop",
                "laya_ext_stats", "laya_ext_attention", "laya_ext_gemm_splitk_static", "laya_ext_hbm_copy",
-               "laya_ext_prof_sequence"]
+               "laya_ext_prof_sequence", "laya_ext_gemm_small", "laya_ext_gemm_small_pick"]
 # every environment variable laya_create reads; Engine() sets the ones it is given for the duration
 # of laya_create only
 ENV_KNOBS = ["LAYA_PRECISION", "LAYA_MAX_TOKENS", "LAYA_PASS_TOKENS", "LAYA_MAX_SEQS", "LAYA_MAX_GATHERED",
@@ -93,6 +93,10 @@ def load_library(path: Optional[str] = None) -> ctypes.CDLL:
     L.laya_ext_gemm_split.restype = ctypes.c_int
     L.laya_ext_gemm_ksplit.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t]
     L.laya_ext_gemm_ksplit.restype = ctypes.c_int
+    L.laya_ext_gemm_small.argtypes = [ctypes.c_int]
+    L.laya_ext_gemm_small.restype = ctypes.c_int
+    L.laya_ext_gemm_small_pick.argtypes = [ctypes.c_int] * 6
+    L.laya_ext_gemm_small_pick.restype = ctypes.c_int
     L.laya_ext_mfma_loop.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_int, ctypes.c_void_p,
                                      ctypes.POINTER(ctypes.c_double)]
     L.laya_ext_mfma_loop.restype = ctypes.c_int
@@ -130,6 +134,15 @@ def gemm_config(lib, cfg: int) -> int:
     prev = lib.laya_ext_gemm_config(cfg)
     if prev == -2:
         raise ValueError("invalid GEMM configuration %d" % cfg)
+    return prev
+
+
+def gemm_small(lib, variant: int) -> int:
+    """Pins a tile of the few-row GEMM kernel for later hook calls (-1: none, 0..4: see laya_ext.h);
+    returns the previous one."""
+    prev = lib.laya_ext_gemm_small(variant)
+    if prev == -2:
+        raise ValueError("invalid few-row GEMM tile %d" % variant)
     return prev
 
 

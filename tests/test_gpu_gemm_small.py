@@ -100,6 +100,86 @@ def test_bf16_passes_of_a_pinned_engine(preset, lens):
     assert np.isfinite(want[0]).all() and np.array_equal(want[0], got[0]) and np.array_equal(want[1], got[1])
 
 
+# the tile that the rule picks for each of SHAPES, store and residual alike: the smallest whose grid is one
+# round of 256 CUs; -1: past the rule's upper end, where the tests above compare the large tiles with themselves
+# (fp32: by the load of the busiest CU)
+PICKS_BF16 = [0, 0, 0, 0, 2, 0, 0, 1, -1, 3, 3, 3, -1]
+
+
+def test_rule_takes_the_shapes():
+    lib = le.load_library()
+    for epi in (0, 1):
+        assert [lib.laya_ext_gemm_small_pick(1, epi, M, N, K, 0) for M, N, K in SHAPES] == PICKS_BF16
+        assert all(0 <= lib.laya_ext_gemm_small_pick(0, epi, M, N, K, 0) <= 3 for M, N, K in SHAPES)
+        assert [lib.laya_ext_gemm_small_pick(1, epi, M, N, K, ks) for M, N, K, ks in SPLITS] == PICKS_SPLIT
+    prev = le.gemm_config(lib, 3)
+    try:
+        assert lib.laya_ext_gemm_small_pick(1, 0, 1, 1024, 1024, 0) == -1
+    finally:
+        le.gemm_config(lib, prev)
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 72, 64), (31, 1024, 192), (33, 72, 2624), (64, 128, 64), (65, 1024, 1024), (129, 136, 1152),
+                                   (513, 1024, 1024)])
+def test_every_tile_gives_the_same_bits(M, N, K):
+    """Each tile on shapes that it does not divide, whatever the rule would pick: bf16 against the large tiles,
+    fp32 against the others (the rule's tile is compared with the generic kernel above)."""
+    import torch
+    lib = le.load_library()
+    for dtype in ("bf16", "fp32"):
+        ops = _operands(M, N, K, dtype, M + N + K)
+        prev = le.gemm_config(lib, 3)
+        try:
+            want = _all(lib, *ops) if dtype == "bf16" else None
+            for v in range(4):
+                le.gemm_small(lib, v)
+                got = _all(lib, *ops)
+                if want is None:
+                    want = got
+                for w, g in zip(want, got):
+                    assert torch.isfinite(g[:M].float()).all() and torch.equal(w, g), (dtype, v)
+                assert all((g[M:] == 7.0).all() for g in got[:3]) and torch.equal(got[3][M:], ops[3][M:])
+            le.gemm_small(lib, 4)
+            with pytest.raises(ValueError):                # 128x64: split-K (and QKV) only
+                le.gemm(lib, ops[0], ops[1], ops[3].clone(), residual=True)
+        finally:
+            le.gemm_small(lib, -1)
+            le.gemm_config(lib, prev)
+
+
+SPLITS = [(M, 1024, K, ks) for M in (1, 67, 513, 1025, 2600) for K, ks in ((1024, 8), (4096, 16), (2624, 7), (2624, 11))]
+PICKS_SPLIT = [0] * 8 + [3] * 4 + [4] * 8
+
+
+@pytest.mark.parametrize("M,N,K,ks", SPLITS)
+def test_split_k_bits_of_the_workspace_path(M, N, K, ks):
+    """Split-K in registers against the slices' reduction (laya_ext_gemm_ksplit): every tile, the 128x64 one in
+    more than one round too, chunks of equal length and with a shorter last one (2624: 41 stages in 6 chunks of 6
+    and one of 5, or 10 of 4 and one of 1)."""
+    import torch
+    lib = le.load_library()
+    ops = _operands(M, N, K, "bf16", M + K + ks)
+    ws = torch.empty(16 << 20, dtype=torch.float32, device="cuda")   # (the engine's 64 MB: several row chunks at M = 2600)
+    prev = le.gemm_ksplit(lib, ks, ws)
+    try:
+        want = _all(lib, *ops)
+        whole = []
+        for v in range(5):
+            le.gemm_small(lib, v)
+            got = _all(lib, *ops)
+            for w, g in zip(want, got):
+                assert torch.isfinite(g[:M].float()).all() and torch.equal(w, g), v
+            assert all((g[M:] == 7.0).all() for g in got[:3]) and torch.equal(got[3][M:], ops[3][M:])
+            whole = got
+        le.gemm_small(lib, -1)
+        le.gemm_ksplit(lib, 0, None)
+        # (the split is there: one sum over all of K has other bits)
+        assert M == 1 or not torch.equal(whole[3], _all(lib, *ops)[3])
+    finally:
+        le.gemm_small(lib, -1)
+        le.gemm_ksplit(lib, prev)
+
+
 def test_fp32_question_alone_and_in_a_batch():
     b = wl.c3(0)
     e = le.Engine(None, ck.cached_checkpoint("large", ln_jitter=0.05), precision="fp32", env={"LAYA_MAX_TOKENS": 16384, "LAYA_GRAPHS": 0})
