@@ -56,6 +56,42 @@ def test_inline_assembly_waits_for_its_own_register_loads(source, tmp_path):
         assert waited, b
 
 
+def _kernels(asm):
+    """(name, total VGPRs, spilled registers, scratch bytes, LDS bytes) of every kernel of the assembly."""
+    val = lambda b, key: int(re.search(r"\.?" + key + r":\s+(\d+)", b).group(1))
+    for b in re.split(r"\n  - ", asm[asm.index("amdhsa.kernels:"):])[1:]:
+        name = re.search(r"\.name:\s+(\S+)", b)
+        if name and "vgpr_count" in b:
+            yield (name.group(1), val(b, "vgpr_count"), val(b, "vgpr_spill_count") + val(b, "sgpr_spill_count"),
+                   val(b, "private_segment_fixed_size"), val(b, "group_segment_fixed_size"))
+
+
+@needs_hipcc
+def test_few_tile_and_few_row_kernels_fit_their_occupancy(tmp_path):
+    """What the launch rules of the small kernels rest on: no spills; three k_attention_narrow workgroups a CU
+    (160 KB of LDS; 16 queries a wave, so 3 or 6 waves a SIMD within 512 / 3 or 512 / 6 registers); two
+    k_attention_f32 workgroups of 4 waves a CU when they split keys, four of whole tiles; k_gemm_small with
+    one workgroup a CU in bf16, two in fp32 but for its smallest tile (32x16: a grid of at most one a CU)."""
+    lds = 160 * 1024
+    found = {"narrow": 0, "f32": 0, "small": 0}
+    for name, vgpr, spill, scratch, l in _kernels(_device_asm("kernels_attn.hip", tmp_path)):
+        if "k_attention_narrow" in name:
+            found["narrow"] += 1
+            assert (spill, scratch) == (0, 0) and 3 * l <= lds and vgpr <= (80 if "ILi8E" in name else 168), (name, vgpr, l)
+        elif "k_attention_f32" in name:
+            found["f32"] += 1
+            n = 2 if "ILb1E" in name else 4
+            assert (spill, scratch) == (0, 0) and n * l <= lds and vgpr <= 512 // n, (name, vgpr, l)
+    for name, vgpr, spill, scratch, l in _kernels(_device_asm("kernels_gemm_small.hip", tmp_path)):
+        if "k_gemm_small" in name:
+            found["small"] += 1
+            n = 1 if "IfLi" not in name or "Li32ELi16E" in name else 2
+            assert (spill, scratch) == (0, 0) and n * l <= lds and vgpr <= 256, (name, vgpr, l)
+    # bf16 tiles x epilogues, plain and split: stores and residuals of five tiles (unsplit: four), QKV of three,
+    # GeGLU of two; fp32: stores and residuals of four tiles, QKV and GeGLU of two
+    assert found == {"narrow": 4, "f32": 2, "small": 2 * 5 + 2 * 4 + 3 + 2 + 2 * 4 + 2 * 2}, found
+
+
 @pytest.mark.skipif(not (os.path.exists(HIPCC) or shutil.which(HIPCC)), reason="hipcc not available")
 def test_attention_kernels_fit_their_occupancy(tmp_path):
     out = tmp_path / "attn.s"
