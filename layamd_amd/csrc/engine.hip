@@ -360,7 +360,8 @@ struct Engine : EngineIface {
     // head's norm1 and, but for the last head layer (gathered rows), norm2.  Off by default: on
     // MI355X at 9.5k rows the residual GEMMs' extra outputs (+3.5 us), the row-statistics kernels
     // (4.8 us) and the consumers' per-element fold (+2.6 to +5 us) cost more than the 12.7 us
-    // LayerNorm kernels they replace.
+    // LayerNorm kernels they replace, and in small passes the folded GEMMs keep the large tiles (128
+    // rows 1226 | 2049 us a pass with the fold, 4096 rows 4671 | 4707).
     fold_ln = sizeof(T) == 2 && D % 64 == 0 && D <= 2048 && env_int("LAYA_LN_FOLD", 0) != 0;
     latency = sizeof(T) == 2 && env_int("LAYA_LATENCY", 0) != 0;
     enc.resize(cfg.n_layers);
@@ -610,14 +611,20 @@ struct Engine : EngineIface {
   // tiles these N = 1024 GEMMs have, instead of walking all of K on a few CUs.  The chunking
   // depends only on K, so every row's result is the same in every batch (and differs from the
   // default engine's in the last bits: the partial sums are added in chunk order).  Larger
-  // passes pay for the fp32 partials: the mode is for latency-bound serving of small batches.
+  // passes pay for the fp32 partials.  The mode dates from before the few-row GEMM kernel, which puts
+  // as many CUs on these GEMMs without splitting K; its own split GEMMs still run on the large tiles
+  // (partials_only), so that the default engine is the faster one at every size (us per pass, default |
+  // this: 128 tokens 1226 | 1341, 512 1716 | 1903, 4 x 512 2952 | 3233).
   // When a pass's partial products fit the workspace in one piece, the GEMM only writes them and
   // the LayerNorm that follows adds them to x (in the reduction's order, so the same bits) before
   // normalising: no reduction launch, and x is read and written once instead of twice.
   static constexpr int kLatencyStages = 4;
   bool latency = false;
   // Bf16 passes of up to kPrefetchRows rows fetch weights ahead (Prefetch) when the encoder's do not fit the
-  // memory-side cache of 256 MB, from which the next pass would read them again.  us per pass without | with:
+  // memory-side cache of 256 MB, from which the next pass would read them again: Wqkv and Wmo always, Wo and
+  // Wi (half of a layer's bytes) where the attention launch before them runs k_attention_narrow, that is not in
+  // passes of many short questions (large model: more than 48 sliding tiles, 32 global ones), and nothing of
+  // the head's two layers.  us per pass without | with:
   // large model (686 MB) 16 rows 1249 | 1155, 128 1305 | 1220 (calls with new questions 1313 | 1253), 304 1613 | 1521,
   // 608 1977 | 1840, 2000 3217 | 3152; base shape (218 MB) 640 rows, new questions, 1208 | 1225.  Above, the
   // GEMMs compute for longer than their weights take.  (fp32 is bound by its MFMAs at any size: 128 rows
@@ -668,7 +675,8 @@ struct Engine : EngineIface {
   }
 
   // one GEMM of the pass: listed while the pass is collected for tuning, otherwise launched on the
-  // few-row kernel where its rule takes it (same bits, nothing to tune), else with the measured configuration of its bucket (the analytic planner's where none was measured)
+  // few-row kernel where its rule takes it (same bits, nothing to tune), else with the measured
+  // configuration of its bucket (the analytic planner's where none was measured)
   void gemm(int epi, GemmArgs g, hipStream_t st) {
     if (collecting) { collecting->emplace_back(epi, g); return; }
     if (pin_cfg < 0 && launch_gemm_small<T>(epi, g, st)) return;

@@ -6,9 +6,10 @@ namespace laya {
 
 // Runs the GEMM on the few-row kernel when its rule takes the shape (bf16: rows few enough that the
 // large tiles of launch_gemm leave most of the chip idle; fp32: any number; aligned operands, no
-// LayerNorm fold) and returns true; otherwise launches nothing and returns false.  Every output is the one launch_gemm gives, bit
-// for bit: the K order, the split-K chunks (GemmArgs::ksplit) and the epilogue's arithmetic are the
-// same.  A pinned tile configuration (gemm_config) keeps launch_gemm.
+// LayerNorm fold, no partials left in the workspace) and returns true; otherwise launches nothing and
+// returns false.  Every output is the one launch_gemm gives, bit for bit: the K order, the split-K
+// chunks (GemmArgs::ksplit) and the epilogue's arithmetic are the same.  A pinned tile configuration
+// (gemm_config) keeps launch_gemm.
 template <typename T>
 bool launch_gemm_small(int epi, const GemmArgs& a, hipStream_t st);
 

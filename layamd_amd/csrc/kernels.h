@@ -66,8 +66,9 @@ struct GemmArgs {
   int split_rows = 0, cfg_tail = -1;
   // split-K (bf16 EPI_STORE / EPI_RESID): K in ksplit chunks of whole 64-deep stages (equal when
   // ksplit divides K / 64, else ceil(K / 64 / ksplit) stages each and a shorter last one) whose
-  // fp32 partial products go to the workspace ws (ws_bytes; rows are processed in chunks that fit
-  // it) and are summed in chunk order, then bias, activation or the residual add.  The result of a row depends on ksplit, not
+  // fp32 sums are added in chunk order, then bias, activation or the residual add.  launch_gemm puts
+  // them into the workspace ws (ws_bytes; rows are processed in chunks that fit it), the few-row kernel
+  // keeps them in registers.  The result of a row depends on ksplit, not
   // on M, so a call site that always passes the same ksplit stays independent of the batch.
   int ksplit = 1;
   float* ws = nullptr;

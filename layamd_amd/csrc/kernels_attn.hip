@@ -401,7 +401,8 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4
   // exp2(s * c - m * c) with c = scale * log2(e), one FMA per score.  The running sum of the
   // probabilities is summed over exactly the bf16 values that the PV product uses, two at a time
   // (v_dot2c_f32_bf16 with (1, 1): a bf16 pair's sum added in fp32), into two partial sums per lane
-  // (the even and the odd 16-key steps, which is how k_attention_narrow's lanes hold them): lane l holds the keys 8 (l / 32) .. + 7 of each 16-key step, so a query's sum is lane l's
+  // (the even and the odd 16-key steps, which is how k_attention_narrow's lanes hold them): lane l holds
+  // the keys 8 (l / 32) .. + 7 of each 16-key step, so a query's sum is lane l's
   // plus lane l ^ 32's, taken once at the end.
   float lsum[2] = {0.f, 0.f};
   float m_run = -INFINITY;
@@ -488,12 +489,12 @@ __global__ __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(NW == 4
       const auto hl = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
       mx = fmaxf(__uint_as_float(hl[0]), __uint_as_float(hl[1]));
     }
-    // m_run, the exponent's reference, trails the running max: it moves (to every lane's max, with
-    // the running output and sum rescaled) only when some valid query's max exceeds it by more
-    // than 2^kLazyLog2 in probability, so probabilities stay at most 2^kLazyLog2 and most blocks
-    // skip the 48 multiplies of the rescale.  The first block has nothing to rescale.  Each query
-    // decides for itself (the others' factor is 1), so its result depends on its own keys only, whatever
-    // the tile size and the queries of a wave.
+    // m_run, the exponent's reference, trails the running max: a query's moves to its max (with its
+    // running output and sum rescaled) only when that exceeds it by more than 2^kLazyLog2 in
+    // probability, so probabilities stay at most 2^kLazyLog2, and a wave skips the 48 multiplies of
+    // the rescale in most blocks, where none of its queries moves (the factor of one that does not
+    // move is 1).  The first block has nothing to rescale.  A query's result thus depends on its own
+    // keys only, whatever the tile size and the queries of a wave.
     const bool need = (mx - m_run) * c2 > kLazyLog2;       // (m_run = -inf: +inf, or NaN with no visible key)
     if (first) {
       m_run = mx;

@@ -3,9 +3,10 @@
 // Both operands are K-contiguous (activations [rows, K], weights in their checkpoint [out, in]
 // layout), which is the layout the MFMA operand registers want: a lane holds 8 consecutive K values
 // of one row of each operand, so every fragment is one 16-byte LDS read and no weight is ever
-// transposed.  Two kernels:
+// transposed.  Two kernels (GEMMs of few rows and fp32 ones run on a third, kernels_gemm_small.hip, with
+// the bits of these):
 //
-//   k_gemm_xl  bf16, the engine's path.  256-thread workgroups, tiles from 128x128 to 256x256 on
+//   k_gemm_xl  bf16, the engine's path for many rows.  256-thread workgroups, tiles from 128x128 to 256x256 on
 //              v_mfma_f32_32x32x16_bf16; K advances in 64-deep stages (whole 128-byte lines of
 //              every tile row), filled ahead by LDS DMA (buffer_load ... lds): two stage buffers,
 //              or for 128x128 tiles three A buffers (two workgroups per CU) or four stage buffers
@@ -13,8 +14,8 @@
 //              transposed so each lane holds four consecutive output columns; the epilogue is
 //              staged through LDS and leaves as full-line 16-byte stores.  The engine picks the
 //              tile shape (and an optional row split over two launches) per GEMM by timing.
-//   k_gemm     fp32 operands, and bf16 shapes the tiled kernel cannot take (unaligned N or
-//              strides).  128x128, 64x64 or 32x64 tiles by how many fill the chip, K in 128-byte
+//   k_gemm     fp32 and bf16 operands that neither of the others takes (unaligned N, strides or
+//              outputs; fp32 also with a pinned tile configuration).  128x128, 64x64 or 32x64 tiles by how many fill the chip, K in 128-byte
 //              slices through double-buffered LDS with register prefetch,
 //              v_mfma_f32_16x16x4_f32 / v_mfma_f32_16x16x32_bf16.
 //

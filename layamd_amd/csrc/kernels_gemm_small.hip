@@ -1,11 +1,13 @@
-// GEMMs on few rows for gfx950: C[M,N] = A[M,K] . W[N,K]^T, M up to a few hundred.
+// GEMMs on few rows for gfx950: C[M,N] = A[M,K] . W[N,K]^T.  bf16: as many rows as one round of tiles on
+// the CUs holds (about 1000 at N = 1024, 200 at N = 5248; split-K: any); fp32: any number.
 //
 // What bounds these: one question is 64 to 512 rows, so with the large tiles of kernels_gemm.hip an
 // N = 1024 GEMM is 16 tiles on 256 CUs, and each of those CUs pulls (128 + 64) rows of all of K through
 // its own L1 fill path (about 50 B/clk) and waits out a trip to HBM for the weights whenever its three
-// stages in flight run dry.  Here the tile is small (32x16 to 64x64), so that 100 to 350 workgroups
-// share those bytes, and nearly all of a CU's LDS is a ring of K stages filled by LDS DMA, so that 70
-// to 140 KB are in flight on a CU, which is what a trip to HBM at that rate takes.
+// stages in flight run dry.  Here the tile is small (32x16 to 64x64; 128x64 for QKV and split-K), so that
+// up to one workgroup per CU shares those bytes, and nearly all of a CU's LDS is a ring of K stages filled
+// by LDS DMA, so that 70 to 140 KB are in flight on a CU, which is what a trip to HBM at that rate takes.
+// In fp32 the MFMAs bind, and the same kernel in rings of half the LDS keeps them busy at any M.
 //
 // Same results as kernels_gemm.hip, bit for bit.  bf16: v_mfma_f32_16x16x32_bf16 accumulates each
 // output exactly as two v_mfma_f32_32x32x16_bf16 do (checked on the hardware, and by the tests against

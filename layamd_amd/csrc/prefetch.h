@@ -14,7 +14,8 @@ struct Prefetch {
   void add(int i, const void* w, size_t bytes) { p[i] = w; lines[i] = (uint32_t)(bytes / 128); }
 };
 struct NoPrefetch {};
-constexpr int kPrefetchBlocks = 192;               // of 256 threads: three lines each of the largest weight
+// of 256 threads each, 49152 in all: a line each of the large model's Wqkv, up to two of its Wi (83968)
+constexpr int kPrefetchBlocks = 192;
 __device__ __forceinline__ void prefetch_lines(const Prefetch& f, uint32_t thread, uint32_t threads) {
 #pragma unroll
   for (int a = 0; a < 2; a++) {

@@ -12,8 +12,9 @@ launch and the TFLOP/s on 2 M N K flop.
 times the GEMM microbenchmark shapes instead: M in {512, 16384}, (N, K) in {(3072, 1024),
 (1024, 1024), (5248, 1024), (1024, 2624)}, bf16 and fp32 operands, against torch.mm (hipBLASLt or
 rocBLAS) on the same device.  bf16 tries the planner and every tile configuration (with split-K
-factors 2, 4 and 8 at M = 512 where K allows them) and reports the best; each engine result is checked
-against torch.mm.  Prints a markdown table.
+factors 2, 4 and 8 at M = 512 where K allows them) and reports the best ("default": what laya_ext_gemm
+runs by itself, the few-row kernel with the named tile where its rule takes the shape, otherwise the
+planner's configuration); each engine result is checked against torch.mm.  Prints a markdown table.
 
     python -m layamd_amd.gemm_probe --c3
 
@@ -40,6 +41,7 @@ import time
 from layamd_amd import engine as le
 
 
+SMALL_TILES = ("32x16", "32x32", "32x64", "64x64", "128x64")   # of the few-row kernel
 ENCODER_NK = ((3072, 1024), (1024, 1024), (5248, 1024), (1024, 2624))
 C2_SHAPES = [(M, N, K) for M in (512, 16384) for (N, K) in ENCODER_NK]
 C3_SHAPES = [(9664, N, K) for (N, K) in ENCODER_NK]
@@ -72,7 +74,7 @@ def c2(lib, shapes=C2_SHAPES, dtypes=None):
     dtypes = dtypes or (torch.bfloat16, torch.float32)
     g = torch.Generator(device="cpu").manual_seed(0)
     ws = torch.empty(64 << 20, dtype=torch.float32, device="cuda")   # split-K partials (256 MiB)
-    print("| M | N | K | dtype | torch.mm us | TFLOP/s | engine us | TFLOP/s | engine plan | planner us | max rel err vs torch.mm |")
+    print("| M | N | K | dtype | torch.mm us | TFLOP/s | engine us | TFLOP/s | engine plan | default us | max rel err vs torch.mm |")
     print("|---:|---:|---:|---|---:|---:|---:|---:|---|---:|---:|")
     for (M, N, K) in shapes:
         fl = 2.0 * M * N * K
@@ -104,7 +106,8 @@ def c2(lib, shapes=C2_SHAPES, dtypes=None):
             le.gemm_config(lib, -1)
             le.gemm_ksplit(lib, 0, None)
             t, cfg, ks, err = best
-            plan = "planner" if cfg == -1 else "cfg %d%s" % (cfg, ", split-K %d" % ks if ks > 1 else "")
+            small = lib.laya_ext_gemm_small_pick(1 if dt == torch.bfloat16 else 0, 0, M, N, K, 0)
+            plan = "default%s" % (" (few-row %s)" % SMALL_TILES[small] if small >= 0 else "") if cfg == -1 else "cfg %d%s" % (cfg, ", split-K %d" % ks if ks > 1 else "")
             print("| %d | %d | %d | %s | %.1f | %.0f | %.1f | %.0f | %s | %.1f | %.1e |"
                   % (M, N, K, "bf16" if dt == torch.bfloat16 else "fp32", t_mm, fl / t_mm / 1e6, t, fl / t / 1e6, plan,
                      t_plan, err), flush=True)
