@@ -681,6 +681,10 @@ __global__ __launch_bounds__(64 * NW) void k_attention_narrow(const bf16_t* __re
   const int jlo_all = win ? max(0, tile.q0 + tile.nq - 1 - window_half) : 0;
   const int jhi_all = win ? min(len, tile.q0 + window_half + 1) : len;
 
+  // Q fragments: d = 32 s + 8 g .. + 7
+  const u32x4_t* qa = reinterpret_cast<const u32x4_t*>(Q + (size_t)(base + p) * ldqk + h * 64) + g;
+  u32x4_t qf[2] = {qa[0], qa[4]};
+
   // DMA plan: instruction j of this wave fills rows 8 i .. + 7 of the K block and of the V^T block, i = wave J + j;
   // blocks from `hi` on come from a resource without records (zeros, no traffic), so that every block is J
   // instructions per operand
@@ -715,36 +719,13 @@ __global__ __launch_bounds__(64 * NW) void k_attention_narrow(const bf16_t* __re
   const bf16x2_t one2 = {(__bf16)1.f, (__bf16)1.f};
   const float c2 = scale * 1.44269504088896340736f;
 
-  // Q fragments (d = 32 s + 8 g .. + 7) and the first two blocks.  One asm block issues them, Q first, and waits
-  // for Q, so that the Q registers hold their values when the compiler first sees them (the fetches of the
-  // blocks, 4 J loads, stay in flight).
-  static_assert(NS == 3, "two blocks before the loop");
-  const char* qa = reinterpret_cast<const char*>(Q + (size_t)(base + p) * ldqk + h * 64) + 16 * g;
-  u32x4_t qf[2];
-  {
-    u32x4_t k1 = rK, v1 = rV;
-    if (lo + 64 >= hi) k1[2] = v1[2] = 0u;
-    uint32_t l = l0 + (uint32_t)(wv * J) * 1024u;
-    const uint32_t dk = (uint32_t)lo * (uint32_t)ldqk * 2u, dv = (uint32_t)lo * 2u, nk = (uint32_t)ldqk * 128u;
-#define ATTN_Q2 "global_load_dwordx4 %0, %3, off\n\tglobal_load_dwordx4 %1, %3, off offset:64\n\t"
-    if constexpr (J == 1)
-      asm volatile(ATTN_Q2 ATTN_DMA("8", "4") ATTN_M0("8192") ATTN_DMA("9", "5") ATTN_M0("8192") ATTN_DMA("10", "6")
-                   ATTN_M0("8192") ATTN_DMA("11", "7") "s_waitcnt vmcnt(4)"
-                   : "=&v"(qf[0]), "=&v"(qf[1]), "+{m0}"(l)
-                   : "v"(qa), "s"(rK), "s"(rV), "s"(k1), "s"(v1), "v"(kvo[0] + dk), "v"(vvo[0] + dv), "v"(kvo[0] + dk + nk),
-                     "v"(vvo[0] + dv + 128u)
-                   : "memory", "scc");
-    else
-      asm volatile(ATTN_Q2 ATTN_DMA("8", "4") ATTN_M0("8192") ATTN_DMA("9", "5") ATTN_M0("-7168") ATTN_DMA("10", "4")
-                   ATTN_M0("8192") ATTN_DMA("11", "5") ATTN_M0("7168") ATTN_DMA("12", "6") ATTN_M0("8192") ATTN_DMA("13", "7")
-                   ATTN_M0("-7168") ATTN_DMA("14", "6") ATTN_M0("8192") ATTN_DMA("15", "7") "s_waitcnt vmcnt(8)"
-                   : "=&v"(qf[0]), "=&v"(qf[1]), "+{m0}"(l)
-                   : "v"(qa), "s"(rK), "s"(rV), "s"(k1), "s"(v1), "v"(kvo[0] + dk), "v"(vvo[0] + dv), "v"(kvo[J - 1] + dk),
-                     "v"(vvo[J - 1] + dv), "v"(kvo[0] + dk + nk), "v"(vvo[0] + dv + 128u), "v"(kvo[J - 1] + dk + nk),
-                     "v"(vvo[J - 1] + dv + 128u)
-                   : "memory", "scc");
-#undef ATTN_Q2
-  }
+#pragma unroll
+  for (int i = 0; i < NS - 1; i++) fetch(lo + 64 * i, i);
+  // The compiler waits for Q here, and with it for the fetches, which it does not see: 0.04 us more a launch than
+  // waiting for Q alone (3.87 -> 3.91 at one question of 128 tokens), which only loads in assembly could, with
+  // registers that it takes as written while they are in flight.  (Q and the fetches in one assembly block that
+  // waits for Q: 3.95, because Q is then issued after the plan above.)
+  asm volatile("" : "+v"(qf[0]), "+v"(qf[1]));
 
   const int krow = 8 * (l16 >> 2) + (l16 & 3);
   int buf = 0;
