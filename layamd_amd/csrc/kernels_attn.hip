@@ -681,17 +681,23 @@ __global__ __launch_bounds__(64 * NW) void k_attention_narrow(const bf16_t* __re
   const int jlo_all = win ? max(0, tile.q0 + tile.nq - 1 - window_half) : 0;
   const int jhi_all = win ? min(len, tile.q0 + window_half + 1) : len;
 
-  // Q fragments: d = 32 s + 8 g .. + 7
-  const u32x4_t* qa = reinterpret_cast<const u32x4_t*>(Q + (size_t)(base + p) * ldqk + h * 64) + g;
-  u32x4_t qf[2] = {qa[0], qa[4]};
+  // Q fragments (d = 32 s + 8 g .. + 7) by LDS DMA too, each lane its own two chunks, into the ring's last block,
+  // which the loop fills only after they are in registers.  In flight under the plan below.  (Loads into
+  // registers would have to be in assembly, or the wait for them would be one for the fetches too: 1222 -> 1227 us
+  // a pass of 128 tokens, 1711 -> 1723 of 512.)
+  const u32x4_t rQ = attn_rsrc(Q, (uint32_t)((size_t)kv_rows * ldqk * 2));
+  const uint32_t l0 = lds_addr_a(L);
+  const int wv = __builtin_amdgcn_readfirstlane(wave);
+#pragma unroll
+  for (int s = 0; s < 2; s++)
+    attn_dma16(rQ, l0 + (NS - 1) * 16384u + (uint32_t)(2 * wv + s) * 1024u,
+               ((uint32_t)(base + p) * (uint32_t)ldqk + (uint32_t)(h * 64 + 32 * s + 8 * g)) * 2u);
 
   // DMA plan: instruction j of this wave fills rows 8 i .. + 7 of the K block and of the V^T block, i = wave J + j;
   // blocks from `hi` on come from a resource without records (zeros, no traffic), so that every block is J
   // instructions per operand
   const u32x4_t rK = attn_rsrc(K, (uint32_t)((size_t)kv_rows * ldqk * 2));
   const u32x4_t rV = attn_rsrc(Vt, (uint32_t)((size_t)vt_rows * ldv * 2));
-  const uint32_t l0 = lds_addr_a(L);
-  const int wv = __builtin_amdgcn_readfirstlane(wave);
   uint32_t kvo[J], vvo[J];
 #pragma unroll
   for (int j = 0; j < J; j++) {
@@ -721,11 +727,10 @@ __global__ __launch_bounds__(64 * NW) void k_attention_narrow(const bf16_t* __re
 
 #pragma unroll
   for (int i = 0; i < NS - 1; i++) fetch(lo + 64 * i, i);
-  // The compiler waits for Q here, and with it for the fetches, which it does not see: 0.04 us more a launch than
-  // waiting for Q alone (3.87 -> 3.91 at one question of 128 tokens), which only loads in assembly could, with
-  // registers that it takes as written while they are in flight.  (Q and the fetches in one assembly block that
-  // waits for Q: 3.95, because Q is then issued after the plan above.)
-  asm volatile("" : "+v"(qf[0]), "+v"(qf[1]));
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * 2 * J) : "memory");   // this wave's Q has landed
+  const u32x4_t* lq = reinterpret_cast<const u32x4_t*>(L) + (NS - 1) * 1024 + wave * 128 + lane;
+  u32x4_t qf[2] = {lq[0], lq[64]};
+  asm volatile("" : "+v"(qf[0]), "+v"(qf[1]));              // read here (in the loop's first block: 12.0 -> 12.4 us for 1024 keys)
 
   const int krow = 8 * (l16 >> 2) + (l16 & 3);
   int buf = 0;
