@@ -522,7 +522,9 @@ static int small_cus() {
 // fp32 is bound by the fp32 MFMA rate, so there the rule weighs the tiles of the busiest CU, at any M:
 //   N 1024, K 2624, residual:  M 128 15.3 | 59.2   512 28.4 | 58.6   1031 64.9 | 104   9664 406 | 678
 //   QKV, N 3072, K 1024:       M 128 13.9 | 28.6   512 32.9 | 44.1   1031 67.3 | 81.6  9664 477 | 564
-// (9664 x 1024 x 2624: 128 of the 152 TFLOP/s that a large fp32 product reaches on this chip).
+// (9664 x 1024 x 2624: 128 of the 152 TFLOP/s that a large fp32 product reaches on this chip.  Against 128x128
+// tiles in whole rounds, residual: 16384 x 1024 x 1024 277 | 297; 20 plain stores in a row, at the power limit,
+// 326 | 317.)
 // 128x64 tiles only gain where the large tiles have none (QKV needs BM <= BN there) or write partial
 // products to memory (split-K; there also in more than one round).
 template <typename T>
