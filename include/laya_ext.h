@@ -107,14 +107,14 @@ int laya_ext_gemm_ksplit(int ks, void* ws, size_t ws_bytes);
 /* The few-row GEMM kernel's tiles: 0..4 are 32x16, 32x32, 32x64, 64x64 and 128x64 (fp32: the first
  * four).  laya_ext_gemm_small_pick gives the one that laya_ext_gemm runs for this type, epilogue and
  * shape with aligned operands, or -1 where the call runs another kernel; with a split-K factor
- * (ksplit > 1, bf16), the one that the engine runs for such a GEMM (laya_ext_gemm itself keeps the
+ * (ksplit 2..64, bf16), the one that the engine runs for such a GEMM (laya_ext_gemm itself keeps the
  * workspace path for a pinned factor).  No launch; needs no GPU.
- * laya_ext_gemm_small makes every later laya_ext_gemm call run that tile, process-wide, with the
- * split-K factor of laya_ext_gemm_ksplit if one is pinned, and return -1 where it does not fit (128x64:
- * split-K only); -1 removes the pin.  Results are the same bits in every case.  Returns the previous
- * setting, or -2 for an invalid value. */
+ * laya_ext_gemm_small launches (does not wait for) that tile on laya_ext_gemm's operands, with K in
+ * ksplit chunks as laya_ext_gemm_ksplit has them (0 or 1: whole), without a workspace.  Returns 0, or -1
+ * where the tile does not take the call (128x64: split-K only).  Results are laya_ext_gemm's, bit for bit. */
 int laya_ext_gemm_small_pick(int dtype, int epi, int M, int N, int K, int ksplit);
-int laya_ext_gemm_small(int variant);
+int laya_ext_gemm_small(int dtype, int epi, const void* A, const void* W, void* C, const float* bias, int act, int M, int N,
+                        int K, int ksplit, int tile, void* stream);
 
 /* laya_ext_gemm's split-K path (bf16 operands, epi 0 store or 1 fp32 residual update, as for
  * laya_ext_gemm with laya_ext_gemm_ksplit(ksplit, ...)), allocating nothing: the fp32 partial

@@ -1101,7 +1101,6 @@ int laya_ext_prof_sequence(void* h, int* stages, int cap) {
 static float* g_ext_ws = nullptr;          // split-K workspace of laya_ext_gemm (caller's memory)
 static size_t g_ext_ws_bytes = 0;
 static int g_ext_ks = 0;                   // split-K factor pinned with it
-static int g_ext_small = -1;               // few-row variant pinned by laya_ext_gemm_small (-1: none)
 
 // The measurement hooks run inside the caller's process, which shares the HIP runtime (and its
 // per-thread last error) with the caller: a stale error that the caller's own HIP calls left must
@@ -1150,18 +1149,11 @@ int laya_ext_gemm(int dtype, int epi, const void* A, const void* W, void* C, con
   // a pinned split-K factor runs in the caller's workspace (laya_ext_gemm_ksplit)
   g.ws = g_ext_ws;
   g.ws_bytes = g_ext_ws_bytes;
-  const int e = epi == 0 ? EPI_STORE : EPI_RESID, small = g_ext_small;
-  if (small >= 0) {
-    if (dtype == 1 && g_ext_ks > 1) g.ksplit = g_ext_ks;
-    if (!(dtype == 0 ? gemm_small_fits<float>(e, g, small) : gemm_small_fits<bf16_t>(e, g, small))) return -1;
-  }
   hipEvent_t a, b;
   if (ms) { LAYA_HIP(hipEventCreate(&a)); LAYA_HIP(hipEventCreate(&b)); LAYA_HIP(hipEventRecord(a, st)); }
   for (int i = 0; i < iters; i++) {
-    if (small >= 0) {
-      if (dtype == 0) launch_gemm_small_variant<float>(e, g, small, st);
-      else launch_gemm_small_variant<bf16_t>(e, g, small, st);
-    } else if (dtype == 0) {
+    const int e = epi == 0 ? EPI_STORE : EPI_RESID;
+    if (dtype == 0) {
       if (!launch_gemm_small<float>(e, g, st)) launch_gemm<float>(e, g, st);
     } else if (g_ext_ks > 1 || !launch_gemm_small<bf16_t>(e, g, st)) {
       launch_gemm<bf16_t>(e, g, st);
@@ -1176,21 +1168,37 @@ int laya_ext_gemm(int dtype, int epi, const void* A, const void* W, void* C, con
   LAYA_HIP(hipGetLastError());
   return 0;
 }
-int laya_ext_gemm_small(int variant) {
-  if (variant < -1 || variant >= laya::kSmallVariants) return -2;
-  const int prev = g_ext_small;
-  g_ext_small = variant;
-  return prev;
+// the arguments of a laya_ext_gemm call on the few-row kernel, which needs no workspace to split K (ws marks
+// the split as allowed and is not read)
+static laya::GemmArgs small_args(int epi, const void* A, const void* W, void* C, const float* bias, int act, int M, int N,
+                                 int K, int ksplit) {
+  static float no_ws;
+  laya::GemmArgs g;
+  g.A = A; g.lda = K; g.W = W; g.ldw = K; g.M = M; g.N = N; g.K = K; g.bias = bias; g.act = act;
+  if (epi == 0) { g.C = C; g.ldc = N; } else { g.X = (float*)C; g.ldx = N; }
+  if (ksplit > 1) { g.ksplit = ksplit; g.ws = &no_ws; }
+  return g;
 }
 int laya_ext_gemm_small_pick(int dtype, int epi, int M, int N, int K, int ksplit) {
   using namespace laya;
-  if ((dtype != 0 && dtype != 1) || (epi != 0 && epi != 1)) return -1;
-  GemmArgs g;                              // (null operands: aligned ones)
-  g.lda = K; g.ldw = K; g.M = M; g.N = N; g.K = K; g.ldc = N; g.ldx = N;
-  float ws;
-  if (ksplit > 1) { g.ksplit = ksplit; g.ws = &ws; }
+  if ((dtype != 0 && dtype != 1) || (epi != 0 && epi != 1) || ksplit < 0 || ksplit > 64) return -1;
+  const GemmArgs g = small_args(epi, nullptr, nullptr, nullptr, nullptr, ACT_NONE, M, N, K, ksplit);
   const int e = epi == 0 ? EPI_STORE : EPI_RESID;
   return dtype == 0 ? gemm_small_pick<float>(e, g) : gemm_small_pick<bf16_t>(e, g);
+}
+int laya_ext_gemm_small(int dtype, int epi, const void* A, const void* W, void* C, const float* bias, int act, int M, int N,
+                        int K, int ksplit, int tile, void* stream) {
+  using namespace laya;
+  if ((dtype != 0 && dtype != 1) || (epi != 0 && epi != 1) || act < 0 || act > 2 || ksplit < 0 || ksplit > 64 || !A || !W || !C)
+    return -1;
+  const GemmArgs g = small_args(epi, A, W, C, bias, act, M, N, K, ksplit);
+  const int e = epi == 0 ? EPI_STORE : EPI_RESID;
+  if (!(dtype == 0 ? gemm_small_fits<float>(e, g, tile) : gemm_small_fits<bf16_t>(e, g, tile))) return -1;
+  (void)hipGetLastError();
+  if (dtype == 0) launch_gemm_small_variant<float>(e, g, tile, (hipStream_t)stream);
+  else launch_gemm_small_variant<bf16_t>(e, g, tile, (hipStream_t)stream);
+  LAYA_HIP(hipGetLastError());
+  return 0;
 }
 const char* laya_ext_precision(void* h) { return E(h)->precision(); }
 

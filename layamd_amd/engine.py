@@ -93,7 +93,7 @@ def load_library(path: Optional[str] = None) -> ctypes.CDLL:
     L.laya_ext_gemm_split.restype = ctypes.c_int
     L.laya_ext_gemm_ksplit.argtypes = [ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t]
     L.laya_ext_gemm_ksplit.restype = ctypes.c_int
-    L.laya_ext_gemm_small.argtypes = [ctypes.c_int]
+    L.laya_ext_gemm_small.argtypes = ([ctypes.c_int] * 2 + [ctypes.c_void_p] * 4 + [ctypes.c_int] * 6 + [ctypes.c_void_p])
     L.laya_ext_gemm_small.restype = ctypes.c_int
     L.laya_ext_gemm_small_pick.argtypes = [ctypes.c_int] * 6
     L.laya_ext_gemm_small_pick.restype = ctypes.c_int
@@ -137,13 +137,14 @@ def gemm_config(lib, cfg: int) -> int:
     return prev
 
 
-def gemm_small(lib, variant: int) -> int:
-    """Pins a tile of the few-row GEMM kernel for later hook calls (-1: none, 0..4: see laya_ext.h);
-    returns the previous one."""
-    prev = lib.laya_ext_gemm_small(variant)
-    if prev == -2:
-        raise ValueError("invalid few-row GEMM tile %d" % variant)
-    return prev
+def gemm_small(lib, A, W, C, tile: int, bias=None, act=0, residual=False, ksplit=0):
+    """One launch of the few-row GEMM kernel with the given tile (0..4, see laya_ext.h) on the current stream."""
+    import torch
+    rc = lib.laya_ext_gemm_small(1 if A.dtype == torch.bfloat16 else 0, 1 if residual else 0, A.data_ptr(), W.data_ptr(),
+                                 C.data_ptr(), bias.data_ptr() if bias is not None else None, act, A.shape[0], W.shape[0],
+                                 A.shape[1], ksplit, tile, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    if rc != 0:
+        raise ValueError("few-row GEMM tile %d rejected: M=%d N=%d K=%d" % (tile, A.shape[0], W.shape[0], A.shape[1]))
 
 
 def gemm_split(lib, split_rows: int, cfg_tail: int = -1):

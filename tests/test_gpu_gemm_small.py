@@ -119,6 +119,17 @@ def test_rule_takes_the_shapes():
         le.gemm_config(lib, prev)
 
 
+def _all_tile(lib, A, W, b, X, tile, ksplit=0):
+    """What _all gives, on one tile of the few-row kernel."""
+    import torch
+    M, N = A.shape[0], W.shape[0]
+    out = [torch.full((M + 8, N), 7.0, dtype=A.dtype, device="cuda") for _ in range(3)] + [X.clone(), X.clone()]
+    for C, bias, act, residual in zip(out, (None, b, b, None, b), (0, 1, 2, 0, 0), (False,) * 3 + (True,) * 2):
+        le.gemm_small(lib, A, W, C, tile, bias=bias, act=act, residual=residual, ksplit=ksplit)
+    torch.cuda.synchronize()
+    return out
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 72, 64), (31, 1024, 192), (33, 72, 2624), (64, 128, 64), (65, 1024, 1024), (129, 136, 1152),
                                    (513, 1024, 1024)])
 def test_every_tile_gives_the_same_bits(M, N, K):
@@ -128,23 +139,22 @@ def test_every_tile_gives_the_same_bits(M, N, K):
     lib = le.load_library()
     for dtype in ("bf16", "fp32"):
         ops = _operands(M, N, K, dtype, M + N + K)
-        prev = le.gemm_config(lib, 3)
-        try:
-            want = _all(lib, *ops) if dtype == "bf16" else None
-            for v in range(4):
-                le.gemm_small(lib, v)
-                got = _all(lib, *ops)
-                if want is None:
-                    want = got
-                for w, g in zip(want, got):
-                    assert torch.isfinite(g[:M].float()).all() and torch.equal(w, g), (dtype, v)
-                assert all((g[M:] == 7.0).all() for g in got[:3]) and torch.equal(got[3][M:], ops[3][M:])
-            le.gemm_small(lib, 4)
-            with pytest.raises(ValueError):                # 128x64: split-K (and QKV) only
-                le.gemm(lib, ops[0], ops[1], ops[3].clone(), residual=True)
-        finally:
-            le.gemm_small(lib, -1)
-            le.gemm_config(lib, prev)
+        want = None
+        if dtype == "bf16":
+            prev = le.gemm_config(lib, 3)
+            try:
+                want = _all(lib, *ops)
+            finally:
+                le.gemm_config(lib, prev)
+        for v in range(4):
+            got = _all_tile(lib, *ops, v)
+            want = want or got
+            for w, g in zip(want, got):
+                assert torch.isfinite(g[:M].float()).all() and torch.equal(w, g), (dtype, v)
+            assert all((g[M:] == 7.0).all() for g in got[:3]) and torch.equal(got[3][M:], ops[3][M:])
+        for v in (4, 5, -1):                               # 128x64: split-K (and QKV) only
+            with pytest.raises(ValueError):
+                _all_tile(lib, *ops, v)
 
 
 SPLITS = [(M, 1024, K, ks) for M in (1, 67, 513, 1025, 2600) for K, ks in ((1024, 8), (4096, 16), (2624, 7), (2624, 11))]
@@ -163,21 +173,15 @@ def test_split_k_bits_of_the_workspace_path(M, N, K, ks):
     prev = le.gemm_ksplit(lib, ks, ws)
     try:
         want = _all(lib, *ops)
-        whole = []
-        for v in range(5):
-            le.gemm_small(lib, v)
-            got = _all(lib, *ops)
-            for w, g in zip(want, got):
-                assert torch.isfinite(g[:M].float()).all() and torch.equal(w, g), v
-            assert all((g[M:] == 7.0).all() for g in got[:3]) and torch.equal(got[3][M:], ops[3][M:])
-            whole = got
-        le.gemm_small(lib, -1)
-        le.gemm_ksplit(lib, 0, None)
-        # (the split is there: one sum over all of K has other bits)
-        assert M == 1 or not torch.equal(whole[3], _all(lib, *ops)[3])
     finally:
-        le.gemm_small(lib, -1)
         le.gemm_ksplit(lib, prev)
+    for v in range(5):
+        got = _all_tile(lib, *ops, v, ks)
+        for w, g in zip(want, got):
+            assert torch.isfinite(g[:M].float()).all() and torch.equal(w, g), v
+        assert all((g[M:] == 7.0).all() for g in got[:3]) and torch.equal(got[3][M:], ops[3][M:])
+    # (the split is there: one sum over all of K has other bits)
+    assert M == 1 or not torch.equal(want[3], _all_tile(lib, *ops, 3)[3])
 
 
 def test_fp32_question_alone_and_in_a_batch():
